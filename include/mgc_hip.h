@@ -171,7 +171,10 @@ enum {
     MGC_GEMM_STREAM = 6,   /* short-K streaming kernel: row-major A with K <= 32, or an NHWC image
                               of one channel group with K <= 48; batch 1, no K split, a column
                               bias (or none), activation none / relu / clip */
-    MGC_GEMM_REGISTER = 7  /* register-staged operands: every operand form (gemm_mfma_kernel) */
+    MGC_GEMM_REGISTER = 7, /* register-staged operands: every operand form (gemm_mfma_kernel) */
+    /* mgc_hip_gemm_planes only: fp32 products on the bf16 matrix cores (gemm_split_kernel), by tile */
+    MGC_GEMM_SPLIT_128X128 = 8,
+    MGC_GEMM_SPLIT_128X64 = 9
 };
 
 void mgc_hip_gemm(mgc_hip_exec *x, const mgc_hip_gemm_args *g);
@@ -179,6 +182,29 @@ void mgc_hip_gemm(mgc_hip_exec *x, const mgc_hip_gemm_args *g);
 /* Workspace floats mgc_hip_gemm wants for a GEMM of this shape (0 = none). The emitter asks
  * at compile time and reserves it through the memory planner's workspace hook. */
 long mgc_hip_gemm_workspace(int M, int N, int K, int batch);
+
+/* GEMMs with a constant right-hand side on the bf16 matrix cores, in fp32 precision: B is laid
+ * out once as three bf16 planes whose sums are its elements (24 bits), A is split the same way
+ * when it is loaded, and six bf16 products accumulated in fp32 stand for each fp32 product.
+ * Against 64 bits the result is no further off than mgc_hip_gemm's; infinities, NaN and
+ * operands too small for the split are recomputed in fp32. No counterpart in the reference
+ * (its mgc_gemm packs B for the CPU's caches, mgc_kernels.c:135-180).
+ *
+ *   mgc_hip_gemm_planes_bytes      bytes of the planes of a K x N right-hand side whose GEMMs over M
+ *                                  rows the library would run this way; 0 when it would not
+ *   mgc_hip_gemm_planes_workspace  workspace floats mgc_hip_gemm_planes wants for its K split
+ *   mgc_hip_gemm_make_planes       writes the planes (256-byte aligned device memory) of b, N rows of
+ *                                  K floats with row stride ldb, on x's stream
+ *   mgc_hip_gemm_planes            mgc_hip_gemm with B's planes: takes everything mgc_hip_gemm takes
+ *                                  (g->b still describes B itself) and runs it as mgc_hip_gemm does
+ *                                  where the planes cannot be used (unaligned operands, batches)
+ *   mgc_hip_gemm_planes_layer_norm the same for mgc_hip_gemm_layer_norm (planes may be NULL) */
+long mgc_hip_gemm_planes_bytes(int M, int N, int K);
+long mgc_hip_gemm_planes_workspace(int M, int N, int K);
+void mgc_hip_gemm_make_planes(mgc_hip_exec *x, const float *b, long ldb, int N, int K, void *planes);
+void mgc_hip_gemm_planes(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const void *planes);
+void mgc_hip_gemm_planes_layer_norm(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const void *planes,
+                                    const float *ln_scale, const float *ln_bias, float eps, float *ln_out);
 
 /* Floats of device scratch the library holds per GPU for mgc_hip_gemm_noalloc (32 MiB). */
 #define MGC_HIP_NOALLOC_SCRATCH_FLOATS (1L << 23)
@@ -579,6 +605,19 @@ typedef struct {
  * the weights once and return the device arena and weights pointers. Idempotent. */
 int mgc_hip_model_init(mgc_hip_model *m, const unsigned char *weights_host, unsigned char **A,
                        unsigned char **W);
+
+/* mgc_hip_model_init for a model whose GEMMs read some constant right-hand sides as bf16 planes
+ * (mgc_hip_gemm_planes): when it allocates the model it also lays those planes out, from the
+ * uploaded weights into the arena past what the plan and the scratch area use. Planes i are made of
+ * the n rows of k floats at W + weights_off and start at A + arena_off (256-byte aligned, within
+ * arena_bytes). On failure the model is released again. */
+typedef struct {
+    size_t weights_off, arena_off;
+    int n, k;
+} mgc_hip_planes_entry;
+
+int mgc_hip_model_init_planes(mgc_hip_model *m, const unsigned char *weights_host, unsigned char **A,
+                              unsigned char **W, const mgc_hip_planes_entry *planes, int n_planes);
 /* Host inputs/outputs: H2D copy, replay of the captured hipGraph, D2H copy, synchronize. */
 int mgc_hip_model_run(mgc_hip_model *m, const void *const *inputs, void *const *outputs,
                       unsigned char *A, const unsigned char *W);

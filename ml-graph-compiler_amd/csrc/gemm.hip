@@ -32,227 +32,9 @@
 
 #include <mutex>
 
-#include "mgc_device.h"
+#include "gemm_split.h"
 
 namespace mgc {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
-
-// A operand forms: strided with unit column stride, NHWC image (implicit im2col), generic
-// (register-staged), and a concatenation of a strided matrix (columns < k1) with an NHWC image
-// read as a strided 1 x 1 convolution (columns >= k1).
-enum { AM_VEC = 0, AM_CONV_VEC = 1, AM_GEN = 2, AM_CAT = 3 };
-
-// 16 zero bytes: the load address of every out-of-range operand element.
-__device__ __attribute__((aligned(16))) float g_zero_page[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-
-// Loads through the global address space. Every operand lives in device memory; saying so
-// keeps the compiler from falling back to flat loads, which share a wait counter with LDS.
-typedef const __attribute__((address_space(1))) float gfloat;
-typedef const __attribute__((address_space(1))) f4 gf4;
-__device__ __forceinline__ float ldg(const float *ptr) { return *(gfloat *)ptr; }
-__device__ __forceinline__ f4 ldg4(const float *ptr) { return *(gf4 *)ptr; }
-enum { BD_NK_VEC = 0, BD_KN_VEC = 1, BD_GEN = 2 };
-
-struct GemmDev {
-    int M, N, K;
-    mgc_hip_operand a, b;
-    float *c;
-    long ldc;
-    float alpha, beta;
-    const float *bias;
-    int bias_mode;
-    const float *res;
-    long ldr;
-    int act;
-    float lo, hi;
-    int batch_rank;
-    int bdims[4];
-    long a_bs[4], b_bs[4], c_bs[4], r_bs[4];
-    int split;    // K splits (1 = none)
-    int kchunk;   // K per split, a multiple of 32
-    float *ws;    // split partials [split][M][N]
-    int tiles_m, tiles_n;
-    int vec_out;
-    FastDiv div_ow, div_ohw, div_cg, div_kw;  // A as NHWC image: OW, OH * OW, cg, KW
-    long a_bytes, b_bytes;  // bytes of A and B reachable from a.p / b.p (all batch elements)
-    mgc_hip_operand a2;     // AM_CAT: the image whose 1 x 1 strided window gives columns >= k1
-    int k1;
-    long a2_bytes;
-    int nbatch;   // batch elements
-    int nfull = 0x7fffffff;  // gemm_dma_kernel: workgroups from this id on compute quarter tiles
-};
-
-__device__ __forceinline__ void batch_offsets(const GemmDev &p, int bz, long &ao, long &bo,
-                                              long &co, long &ro) {
-    ao = bo = co = ro = 0;
-    int rem = bz;
-#pragma unroll
-    for (int d = 3; d >= 0; --d) {
-        if (d < p.batch_rank) {
-            int idx = rem % p.bdims[d];
-            rem /= p.bdims[d];
-            ao += idx * p.a_bs[d];
-            bo += idx * p.b_bs[d];
-            co += idx * p.c_bs[d];
-            ro += idx * p.r_bs[d];
-        }
-    }
-}
-
-__device__ __forceinline__ f4 act4(f4 v, int act, float lo, float hi) {
-    switch (act) {
-    case MGC_ACT_RELU:
-        v[0] = v[0] > 0.0f ? v[0] : 0.0f;
-        v[1] = v[1] > 0.0f ? v[1] : 0.0f;
-        v[2] = v[2] > 0.0f ? v[2] : 0.0f;
-        v[3] = v[3] > 0.0f ? v[3] : 0.0f;
-        return v;
-    case MGC_ACT_CLIP:
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = fminf(fmaxf(v[e], lo), hi);
-        return v;
-    case MGC_ACT_GELU:
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = gelu_erf_f(v[e]);
-        return v;
-    case MGC_ACT_GELU_TANH:
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = gelu_tanh_f(v[e]);
-        return v;
-    case MGC_ACT_TANH:
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = tanh_f(v[e]);
-        return v;
-    case MGC_ACT_SIGMOID:
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = sigmoid_f(v[e]);
-        return v;
-    default: return v;
-    }
-}
-
-// Epilogue shared by the GEMM kernels, pass 2: the BM x BN tile, staged in LDS at Cs with row
-// pitch BN + 8 floats, leaves as 16-byte chunks with alpha, bias, residual and activation
-// applied, or raw into the split-K workspace. Each thread owns one fixed 16-byte column chunk
-// of the tile and the rows r0, r0 + RSTEP, ..., so the column bias is read once per thread.
-// Every one of the 256 threads calls it (no barrier inside).
-template <int BM, int BN>
-__device__ __forceinline__ void gemm_lds_to_global(const GemmDev &p, const float *Cs, int m0, int n0, int ks,
-                                                   long co, long ro) {
-    constexpr int LDC = BN + 8;
-    const f4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    const int tid = threadIdx.x;
-    constexpr int C4 = BN / 4;
-    static_assert(256 % C4 == 0, "column chunks must divide the workgroup");
-    constexpr int RSTEP = 256 / C4;
-    constexpr int ITERS = BM / RSTEP;
-    constexpr int G = ITERS < 4 ? ITERS : 4;
-    // Scalars read once: keeps the compiler from copying the argument block to scratch.
-    const float alpha = p.alpha, beta = p.beta, lo = p.lo, hi = p.hi;
-    const float *const bias = p.bias;
-    const int act = p.act, M = p.M, N = p.N;
-    const bool split_out = p.split > 1;
-    float *const cbase = split_out ? p.ws + (long)ks * M * N : p.c + co;
-    const long ldc = split_out ? (long)N : p.ldc;
-    const float *const rbase = (!split_out && p.res) ? p.res + ro : nullptr;
-    const bool vec = split_out ? (N % 4 == 0) : (p.vec_out != 0);
-    const int cl = (tid % C4) * 4;
-    const int col = n0 + cl;
-    const int r0 = tid / C4;
-    const bool col_ok = col < N;
-    const int ncol = col_ok ? min(4, N - col) : 0;
-    const bool full4 = vec && ncol == 4;
-    const int bmode = split_out ? 0 : p.bias_mode;
-    f4 cbias = zero4;
-    if (bmode == 1 && col_ok) {
-        if (full4) {
-            cbias = ldg4(bias + col);
-        } else {
-            for (int e = 0; e < ncol; ++e) cbias[e] = ldg(bias + col + e);
-        }
-    }
-    // pass 2: LDS tile -> epilogue -> memory, 16 bytes per access, G rows per step with their
-    // residual chunks (and row biases) requested together.
-    if (!col_ok) return;
-    const bool pre_res = rbase != nullptr && full4;
-#pragma unroll 1
-    for (int g = 0; g < ITERS; g += G) {
-        f4 rv[G];
-        float rb[G];
-#pragma unroll
-        for (int u = 0; u < G; ++u) {
-            const int row = m0 + r0 + RSTEP * (g + u);
-            const bool ok = row < M;
-            rv[u] = zero4;
-            rb[u] = 0.0f;
-            if (pre_res)
-                rv[u] = ldg4(ok ? rbase + (long)row * p.ldr + col
-                                                         : g_zero_page);
-            if (bmode == 2) rb[u] = ldg(ok ? bias + row : g_zero_page);
-        }
-#pragma unroll
-        for (int u = 0; u < G; ++u) {
-            const int rl = r0 + RSTEP * (g + u);
-            const int row = m0 + rl;
-            if (row >= M) break;
-            f4 v = *reinterpret_cast<const f4 *>(&Cs[rl * LDC + cl]);
-            float *dst = cbase + (long)row * ldc + col;
-            if (!split_out) {
-                v = v * alpha + cbias;
-                if (bmode == 2) v += rb[u];
-                if (pre_res) {
-                    v += beta * rv[u];
-                } else if (rbase) {
-                    const float *src = rbase + (long)row * p.ldr + col;
-                    for (int e = 0; e < ncol; ++e) v[e] += beta * ldg(src + e);
-                }
-                v = act4(v, act, lo, hi);
-            }
-            if (full4) {
-                *reinterpret_cast<f4 *>(dst) = v;
-            } else {
-                for (int e = 0; e < ncol; ++e) dst[e] = v[e];
-            }
-        }
-    }
-}
-
-
-
-
-// The whole epilogue: pass 1 moves the accumulators to LDS (smem, at least BM * (BN + 8)
-// floats, free when this is called), then gemm_lds_to_global.
-template <int BM, int BN, int WGM, int RM, int RN>
-__device__ __forceinline__ void gemm_store_tile(const GemmDev &p, float *smem,
-                                                     const floatx16 (&acc)[RM][RN], int m0, int n0,
-                                                     int ks, long co, long ro) {
-    constexpr int WGN = 4 / WGM;
-    constexpr int WM = BM / WGM;
-    constexpr int WN = BN / WGN;
-    constexpr int LDC = BN + 8;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int wm = wave / WGN, wn = wave - (wave / WGN) * WGN;
-    const int li = lane & 31;
-    const int lh = lane >> 5;
-    // pass 1: registers -> LDS tile. Block (i, j) register r holds tile row
-    // 8 * (r / 4) + 4 * lh + r % 4 and column li of that 32x32 block.
-    float *const Cs = smem;
-#pragma unroll
-    for (int i = 0; i < RM; ++i)
-#pragma unroll
-        for (int j = 0; j < RN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                Cs[(wm * WM + i * 32 + (r >> 2) * 8 + lh * 4 + (r & 3)) * LDC + wn * WN + j * 32 +
-                   li] = acc[i][j][r];
-    __syncthreads();
-    gemm_lds_to_global<BM, BN>(p, Cs, m0, n0, ks, co, ro);
-}
 
 template <int BM, int BN, int WGM, int AMODE, int BMODE>
 __global__ void __launch_bounds__(256) gemm_mfma_kernel(const GemmDev p) {
@@ -528,27 +310,6 @@ __global__ void __launch_bounds__(256) gemm_mfma_kernel(const GemmDev p) {
 
     gemm_store_tile<BM, BN, WGM>(p, smem, acc, m0, n0, ks, co, ro);
 }
-
-// s_waitcnt with only the vector-memory counter constrained (expcnt and lgkmcnt at maximum).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x70 | 0xF00);
-}
-
-// Workgroup barrier for the LDS ring: waits for this wave's own LDS accesses only. The
-// __syncthreads() fence would also wait for every outstanding global load, including the
-// DMA loads of later pipeline stages, and drain the ring at every step.
-__device__ __forceinline__ void barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-typedef __attribute__((address_space(3))) void lds_void;
-
-// 16 bytes at byte offset voff of a buffer resource straight into LDS (lane l of the wave
-// writes lds_base + 16 * l); offsets at or past the resource's size read as zeros.
-__device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t r, unsigned voff, float *lds_base) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds_base, 16, (int)voff, 0, 0, 0);
-}
-
 
 // GEMM / implicit-GEMM convolution for k-contiguous operands (A: strided with unit column
 // stride, or an NHWC image with channel groups divisible by 4; B: packed [N][K]).
@@ -2956,6 +2717,45 @@ static int wave_split_ln(int M, int N, int K, int split) {
     return best;
 }
 
+// Tile and K split of a GEMM with planes of B (gemm_split.hip), or bm 0 where the fp32 kernels are
+// faster. A launch takes as long as its busiest CU, so a tile shape costs ceil(tiles / 256) times
+// one tile; measured per 32-wide stage, a 128 x 128 tile takes 1.8 times a 128 x 64 one (4096 x 3072
+// x 768: 768 tiles 106 us, 1536 tiles 118 us; 25088 x 128 x 1152: 196 tiles 51 us, 392 tiles 53 us).
+// K is split in up to four where the tiles leave CUs idle, at least 256 k a part (more parts were
+// never faster than the fp32 kernels: 256 x 768 x 3072 in eight 20.0 against 20.7 us), and `split` > 0
+// fixes it.
+//
+// The fp32 kernels stay where a launch cannot fill the chip: these tiles are large and a stage is
+// a long chain (load, split, multiply), so they win from three quarters of a round of workgroups
+// on (us, fp32 / split: 2048 x 768 x 768, 192 tiles, 25.5 / 23.7; 512 x 2304 x 768, 144 tiles, 23.5 /
+// 24.1; 1024 x 2304 x 768, 288 tiles, 34.7 / 39.3) and with K of 192 on, or from about 1536 tiles
+// on with shorter K (100352 x 256 x 64 46.4 / 40.3; 100352 x 64 x 64, 784 tiles, 16.5 / 17.8; 4096 x 512
+// x 128, 256 tiles, 9.9 / 11.0).
+static SplitChoice split_choice(int M, int N, int K, long workspace_floats, int split) {
+    const SplitChoice none{0, 0, 0};
+    if (N < 64 || K < 64 || (N + 63) / 64 * 64 > N + N / 4 || (M + 127) / 128 * 128 > M + M / 3) return none;  // padding
+    SplitChoice best = none;
+    double best_cost = 0.0;
+    const int stages = (K + 31) / 32;
+    const int max_split = split > 0 ? split : K / 256 < 4 ? (K / 256 > 1 ? K / 256 : 1) : 4;
+    for (int bn = 64; bn <= 128; bn += 64) {
+        const long tiles = (long)((M + 127) / 128) * ((N + bn - 1) / bn);
+        for (int s = split > 0 ? split : 1; s <= max_split; ++s) {
+            if (s > 1 && split <= 0 && (tiles >= kCUs || (long)s * M * N > workspace_floats)) break;
+            const long wgs = tiles * s, rounds = (wgs + kCUs - 1) / kCUs;
+            if (wgs < kCUs * 3 / 4 || wgs * 10 < rounds * kCUs * 6 || (K < 192 && wgs < 6 * kCUs)) continue;
+            // microseconds: the stages, and a reduction's launch and traffic
+            double cost = (double)rounds * ((stages + s - 1) / s) * (bn == 128 ? 1.33 : 0.74);
+            if (s > 1) cost += 4.0 + (2.0 * s + 1.0) * M * N * 1e-6;
+            if (!best.bm || cost < best_cost) {
+                best = SplitChoice{128, bn, s};
+                best_cost = cost;
+            }
+        }
+    }
+    return best;
+}
+
 // 128 x 32 tiles (four waves stacked along M) instead of 64 x 64 when they pad N less: the
 // pointwise convolutions of MobileNet-style networks have 16 to 160 output channels, where a
 // 64-wide tile leaves up to 3/4 of the matrix-core work and of the epilogue on padding. Only
@@ -2988,9 +2788,46 @@ static int ln_split(int M, int N, int K) {
     return t.split > 1 ? t.split : 2;
 }
 
-static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTail *ln);
+static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTail *ln, const void *planes = nullptr);
 
 extern "C" void mgc_hip_gemm(mgc_hip_exec *x, const mgc_hip_gemm_args *g) { gemm_launch(x, g, nullptr); }
+
+// ---------------------------------------------------------------------------------------------
+// Constant right-hand sides as bf16 planes (gemm_split.hip)
+// ---------------------------------------------------------------------------------------------
+// Blocks of a K x N matrix: 16-k blocks per column block (whole 32-wide stages), column blocks.
+static const long kAnyWorkspace = 0x7fffffffffffffffL;
+static int plane_kblocks(int K) { return (K + 31) / 32 * 2; }
+static int plane_nblocks(int N) { return (N + 31) / 32; }
+static long plane_data_bytes(int N, int K) { return (long)plane_nblocks(N) * plane_kblocks(K) * 3072; }
+
+extern "C" long mgc_hip_gemm_planes_bytes(int M, int N, int K) {
+    if (M < 1 || N < 1 || K < 1) return 0;
+    // alone, or with a LayerNorm tail, which fixes the K split
+    if (!split_choice(M, N, K, kAnyWorkspace, 0).bm && !split_choice(M, N, K, kAnyWorkspace, ln_split(M, N, K)).bm)
+        return 0;
+    const long bytes = plane_data_bytes(N, K);
+    // the planes, then a byte per column (whole blocks); buffer offsets end at 2 GiB
+    return bytes < 0x7fffffffL ? (bytes + plane_nblocks(N) * 32L + 255) / 256 * 256 : 0;
+}
+
+extern "C" long mgc_hip_gemm_planes_workspace(int M, int N, int K) {
+    if (!mgc_hip_gemm_planes_bytes(M, N, K)) return 0;
+    const SplitChoice c = split_choice(M, N, K, kAnyWorkspace, 0);
+    return c.split > 1 ? (long)c.split * M * N : 0;
+}
+
+extern "C" void mgc_hip_gemm_make_planes(mgc_hip_exec *x, const float *b, long ldb, int N, int K, void *planes) {
+    const int kb = plane_kblocks(K), nb = plane_nblocks(N);
+    MGC_LAUNCH(x, split_planes_kernel, dim3(blocks_for((long)kb * nb * 64, 256, 16384)), dim3(256), 0, b, ldb, N, K, kb,
+               nb, static_cast<uint4_t *>(planes));
+    MGC_LAUNCH(x, tiny_columns_kernel, dim3((unsigned)(nb * 32 / 4)), dim3(256), 0, b, ldb, N, K,
+               static_cast<unsigned char *>(planes) + plane_data_bytes(N, K), nb * 32);
+}
+
+extern "C" void mgc_hip_gemm_planes(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const void *planes) {
+    gemm_launch(x, g, nullptr, planes);
+}
 
 // ---------------------------------------------------------------------------------------------
 // mgc_hip_gemm_noalloc: mgc_hip_gemm with the K-split partials in the library's own device
@@ -3084,6 +2921,12 @@ extern "C" long mgc_hip_gemm_layer_norm_workspace(int M, int N, int K) {
 
 extern "C" void mgc_hip_gemm_layer_norm(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const float *ln_scale,
                                         const float *ln_bias, float eps, float *ln_out) {
+    mgc_hip_gemm_planes_layer_norm(x, g, nullptr, ln_scale, ln_bias, eps, ln_out);
+}
+
+extern "C" void mgc_hip_gemm_planes_layer_norm(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const void *planes,
+                                               const float *ln_scale, const float *ln_bias, float eps,
+                                               float *ln_out) {
     if (g->M <= 0) return;
     const int split = ln_split(g->M, g->N, g->K);
     const bool ok = mgc_hip_gemm_layer_norm_supported(g->M, g->N) && g->batch_rank == 0 &&
@@ -3101,7 +2944,7 @@ extern "C" void mgc_hip_gemm_layer_norm(mgc_hip_exec *x, const mgc_hip_gemm_args
     mgc_hip_gemm_args a = *g;
     a.split_k = split;
     const LnTail tail{ln_scale, ln_bias, eps, ln_out};
-    gemm_launch(x, &a, &tail);
+    gemm_launch(x, &a, &tail, planes);
 }
 
 extern "C" void mgc_hip_gemm_dw(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const mgc_hip_dw_args *dw) {
@@ -3356,7 +3199,7 @@ extern "C" void mgc_hip_expand_dw(mgc_hip_exec *x, const mgc_hip_expand_dw_args 
     MGC_LAUNCH(x, kern, dim3((unsigned)((long)a->N * d.slices)), dim3(256), 0, d);
 }
 
-static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTail *ln) {
+static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTail *ln, const void *planes) {
     if (g->M <= 0 || g->N <= 0) return;
     GemmDev p;
     p.M = g->M;
@@ -3485,10 +3328,20 @@ static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTai
         return;
     }
 
+    // The bf16-split kernels read eight k of one window tap at a time and B as planes.
+    const bool split_ok = planes != nullptr && dma_ok && batch == 1 && (am != AM_CONV_VEC || p.a.cg % 8 == 0) &&
+                          plane_data_bytes(p.N, p.K) < kMaxRes;
+
     // The kernel family and K split: the library's choice from the shape, or the caller's
     // (g->kernel, g->split_k), checked against what that family accepts.
     int fam;
-    if (g->kernel == MGC_GEMM_AUTO || ln) {
+    SplitChoice sc{0, 0, 0};
+    if (g->kernel == MGC_GEMM_AUTO && split_ok && g->split_k <= 0)
+        sc = split_choice(p.M, p.N, p.K, g->workspace == nullptr ? 0 : g->workspace_floats, ln ? p.split : 0);
+    if (sc.bm) {
+        fam = sc.bn == 64 ? MGC_GEMM_SPLIT_128X64 : MGC_GEMM_SPLIT_128X128;
+        p.split = sc.split;
+    } else if (g->kernel == MGC_GEMM_AUTO || ln) {
         if (stream_ok && g->split_k <= 0 &&
             (am == AM_VEC ? use_stream(p.M, p.N, p.K) : use_stream_conv(p.M, p.N, p.K))) {
             fam = MGC_GEMM_STREAM;
@@ -3522,8 +3375,12 @@ static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTai
         fam = g->kernel;
         const int split = g->split_k > 1 ? g->split_k : 1;
         const char *why = nullptr;
-        if (fam < MGC_GEMM_TILED || fam > MGC_GEMM_REGISTER)
+        const bool split_fam = fam >= MGC_GEMM_SPLIT_128X128 && fam <= MGC_GEMM_SPLIT_128X64;
+        if (fam < MGC_GEMM_TILED || fam > MGC_GEMM_SPLIT_128X64)
             why = "unknown kernel family";
+        else if (split_fam && !split_ok)
+            why = "the bf16-split kernels need planes of B (mgc_hip_gemm_planes), batch 1, k-contiguous operands below "
+                  "2 GiB and convolution groups of a multiple of 8 channels";
         else if (split > 1 && (batch != 1 || g->workspace == nullptr || g->workspace_floats < (long)split * p.M * p.N))
             why = "a K split needs batch 1 and split_k * M * N floats of workspace";
         else if (fam != MGC_GEMM_REGISTER && fam != MGC_GEMM_STREAM && !dma_ok)
@@ -3556,11 +3413,14 @@ static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTai
     }
     p.kchunk = ((p.K + p.split - 1) / p.split + 31) / 32 * 32;
     if (p.kchunk == 0) p.kchunk = 32;
-    const int bm_t = fam == MGC_GEMM_WSPLIT16 ? 16 : fam == MGC_GEMM_WSPLIT ? 32 : fam == MGC_GEMM_NARROW ? 128 : 64;
-    const int bn_t = fam == MGC_GEMM_WSPLIT16 ? 16 : fam == MGC_GEMM_WSPLIT || fam == MGC_GEMM_NARROW ? 32 : 64;
+    const bool split_fam = fam >= MGC_GEMM_SPLIT_128X128;
+    const int bn_s = fam == MGC_GEMM_SPLIT_128X128 ? 128 : 64;
+    const int bm_t = split_fam ? 128 : fam == MGC_GEMM_WSPLIT16 ? 16 : fam == MGC_GEMM_WSPLIT ? 32 : fam == MGC_GEMM_NARROW ? 128 : 64;
+    const int bn_t = split_fam ? bn_s : fam == MGC_GEMM_WSPLIT16 ? 16 : fam == MGC_GEMM_WSPLIT || fam == MGC_GEMM_NARROW ? 32 : 64;
     p.tiles_m = (p.M + bm_t - 1) / bm_t;
     p.tiles_n = (p.N + bn_t - 1) / bn_t;
-    GemmKernel kern = fam == MGC_GEMM_WSPLIT16 ? pick_wsplit16(am, p.kchunk)
+    GemmKernel kern = split_fam ? nullptr
+                      : fam == MGC_GEMM_WSPLIT16 ? pick_wsplit16(am, p.kchunk)
                       : fam == MGC_GEMM_WSPLIT ? pick_wsplit(am)
                       : fam == MGC_GEMM_NARROW ? pick_dma<128, 32, 4>(am)
                       : fam == MGC_GEMM_QUARTER ? pick_dma_tail(am)
@@ -3574,7 +3434,12 @@ static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTai
         set_error("mgc_hip_gemm_layer_norm: no K split", hipErrorInvalidValue);
         return;
     }
-    MGC_LAUNCH(x, kern, grid, dim3(threads), 0, p);
+    if (split_fam) {
+        MGC_LAUNCH(x, pick_split(am, bn_s), grid, dim3(256), 0, p, static_cast<const unsigned char *>(planes),
+                   plane_data_bytes(p.N, p.K), plane_kblocks(p.K));
+    } else {
+        MGC_LAUNCH(x, kern, grid, dim3(threads), 0, p);
+    }
     if (ln) {
         // a wavefront per row; one-wave workgroups when there are few rows, to spread them over CUs
         const int rows_per_block = p.M >= 1024 ? 4 : 1;

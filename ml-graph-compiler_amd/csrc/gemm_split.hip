@@ -1,0 +1,377 @@
+// fp32 GEMM and implicit-GEMM convolution on the bf16 matrix cores, with 24-bit operands.
+//
+// gfx950 multiplies fp32 at 157 TFLOP/s (v_mfma_f32_32x32x2_f32) and bf16 at 2.5 PFLOP/s. An fp32
+// number is the exact sum of three bf16 numbers, x = h + m + l (each the round-to-nearest bf16 of
+// what the ones before leave: 8 + 8 + 8 significant bits), so
+//   a b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh) + O(2^-25 |a b|)
+// is six bf16 products, summed in fp32 by v_mfma_f32_32x32x16_bf16: 6 x 32 cycles for 16 k of a
+// 32 x 32 block against 8 x 64 cycles in fp32, a ceiling of 416 TFLOP/s. The dropped products
+// (am bl, al bm, al bl) are below the rounding of one fp32 product. The leading products and the
+// five corrections have an accumulator each, so the corrections are not rounded at the size of
+// the whole sum, and the leading sum is rounded once per 16 k instead of once per product:
+// against 64 bits a 768-long dot product of normal numbers is 1.5e-7 off (fp32 MFMA: 4.8e-7), a
+// 4608-long one 4.3e-7 (1.2e-6).
+//
+// What the split cannot carry is recomputed in fp32 from the operands, element by element, in the
+// epilogue: sums that are not finite (an infinite or NaN operand, or an overflow: inf - inf in the
+// split, or inf times a zero part, makes a NaN where fp32 has an infinity) and the rows and
+// columns of operands that are all below 2^-95, whose low parts fall under the bf16 range.
+#include "gemm_split.h"
+
+namespace mgc {
+
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef unsigned uint2_t __attribute__((ext_vector_type(2)));
+
+// Two floats rounded to nearest bf16, packed (v_cvt_pk_bf16_f32).
+__device__ __forceinline__ unsigned pack_bf16(float x, float y) {
+    const f2 v = {x, y};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf2));
+}
+
+// Two floats as three packed bf16 pairs whose exact sums they are.
+__device__ __forceinline__ void split3(float x, float y, unsigned &h, unsigned &m, unsigned &l) {
+    h = pack_bf16(x, y);
+    x -= __uint_as_float(h << 16);
+    y -= __uint_as_float(h & 0xffff0000u);
+    m = pack_bf16(x, y);
+    x -= __uint_as_float(m << 16);
+    y -= __uint_as_float(m & 0xffff0000u);
+    l = pack_bf16(x, y);
+}
+
+// 16 bytes at byte offset voff of a buffer resource; zeros at or past its end.
+__device__ __forceinline__ f4 buf_load4(__amdgpu_buffer_rsrc_t r, unsigned voff) {
+    return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, 0, 0));
+}
+
+// Workgroup barrier of a stage: this wave's loads but the last N have landed, its LDS reads too.
+// One statement, so that no load moves across the wait that counts it.
+template <int N>
+__device__ __forceinline__ void barrier_stage() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// One element's sum over [kbeg, kend) in fp32, straight from the operands.
+template <int AMODE>
+__device__ __forceinline__ float dot_fp32(const GemmDev &p, const float *abase, const float *bbase, int row, int col,
+                                          int kbeg, int kend) {
+    float sum = 0.0f;
+    const mgc_hip_operand &img = AMODE == AM_CAT ? p.a2 : p.a;
+    int n = 0, oh = 0, ow = 0;
+    if (AMODE != AM_VEC) {
+        n = fdiv(row, p.div_ohw);
+        const int rr = row - n * img.OH * img.OW;
+        oh = fdiv(rr, p.div_ow);
+        ow = rr - oh * img.OW;
+    }
+#pragma unroll 1
+    for (int k = kbeg; k < kend; ++k) {
+        float a;
+        if (AMODE == AM_CONV_VEC) {
+            const int t = fdiv(k, p.div_cg);
+            const int kh = fdiv(t, p.div_kw);
+            const int ih = oh * p.a.SH - p.a.PT + kh * p.a.DH;
+            const int iw = ow * p.a.SW - p.a.PL + (t - kh * p.a.KW) * p.a.DW;
+            const bool ok = (unsigned)ih < (unsigned)p.a.H && (unsigned)iw < (unsigned)p.a.W;
+            a = ldg(ok ? abase + (((long)n * p.a.H + ih) * p.a.W + iw) * p.a.C + (k - t * p.a.cg) : g_zero_page);
+        } else if (AMODE == AM_CAT && k >= p.k1) {
+            a = ldg(p.a2.p + (((long)n * p.a2.H + oh * p.a2.SH) * p.a2.W + ow * p.a2.SW) * p.a2.C + (k - p.k1));
+        } else {
+            a = ldg(abase + (long)row * p.a.rs + k);
+        }
+        sum = fmaf(a, ldg(bbase + (long)col * p.b.cs + k), sum);
+    }
+    return sum;
+}
+
+// Split the constant right-hand side b ([N][K] with row stride ldb) into planes. One thread per
+// 8 consecutive k of one column (16 bytes of each plane); padding is written as zeros. mark[n] is
+// set (a byte, cleared before) when column n has an element of 2^-95 or more, see tiny_columns.
+__global__ void __launch_bounds__(256) split_planes_kernel(const float *b, long ldb, int N, int K, int kb, int nb,
+                                                           uint4_t *planes) {
+    const long total = (long)nb * kb * 64;
+    for (long t = blockIdx.x * 256L + threadIdx.x; t < total; t += gridDim.x * 256L) {
+        const int lane = (int)(t & 63);
+        const long block = t >> 6;  // (column block, 16-k block)
+        const int n = (int)(block / kb) * 32 + (lane & 31);
+        const int k = (int)(block % kb) * 16 + (lane >> 5) * 8;
+        uint4_t h, m, l;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float x = n < N && k + 2 * e < K ? b[n * ldb + k + 2 * e] : 0.0f;
+            const float y = n < N && k + 2 * e + 1 < K ? b[n * ldb + k + 2 * e + 1] : 0.0f;
+            unsigned u, v, w;
+            split3(x, y, u, v, w);
+            h[e] = u;
+            m[e] = v;
+            l[e] = w;
+        }
+        uint4_t *const dst = planes + block * 192 + lane;
+        dst[0] = h;
+        dst[64] = m;
+        dst[128] = l;
+    }
+}
+
+// flags[n] = 1 when every element of column n of b is below 2^-95 and not all are zero. One wave
+// per column.
+__global__ void __launch_bounds__(256) tiny_columns_kernel(const float *b, long ldb, int N, int K,
+                                                           unsigned char *flags, int nflags) {
+    const int n = (int)((blockIdx.x * 256L + threadIdx.x) >> 6), lane = threadIdx.x & 63;
+    if (n >= nflags) return;
+    float most = 0.0f;
+    if (n < N)
+        for (int k = lane; k < K; k += 64) most = fmaxf(most, fabsf(b[(long)n * ldb + k]));
+    most = wave_max(most);
+    if (lane == 0) flags[n] = most > 0.0f && most < 0x1p-95f;
+}
+
+// A workgroup of WAVES waves owns a tile of 32 WAVES rows x 32 RN columns; each wave owns 32 rows and
+// all the columns. K advances 32 per stage (two MFMA depths of 16).
+//
+//  * A: a lane's MFMA operand is 8 consecutive k of one row, so the wave loads its own rows' fp32
+//    straight into registers two stages ahead (two 16-byte loads per 16 k through a buffer
+//    resource; masked elements read as zero) and splits them there: each element is split once
+//    per column tile, and A never goes through LDS.
+//  * B: planes split once when the weights are laid out, in fragment order (for a block of 32
+//    columns and 16 k the three planes' 64 lanes x 16 bytes), so a stage is copied to LDS by
+//    linear 1 KB DMA instructions and read back as linear 16-byte fragments without bank
+//    conflicts. A ring of R stages, one barrier per stage, loads two stages ahead.
+//
+// A wave's 32 x 128 part has 2 x 64 accumulator registers, which two waves per SIMD (two
+// workgroups per CU) allow.
+template <int RN, int WAVES, int R, int AMODE>
+__global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
+    gemm_split_kernel(const GemmDev p, const unsigned char *planes, long plane_bytes, int kblocks) {
+    constexpr int BK = 32;
+    constexpr int BM = 32 * WAVES, BN = 32 * RN;
+    constexpr int SLOT = RN * 6 * 1024;             // bytes of one stage of B
+    constexpr int DMA = RN * 6 / WAVES;             // 1 KB copies per wave and stage
+    static_assert(RN * 6 % WAVES == 0, "copies divide among the waves");
+    constexpr int EPI = BM * (BN + 8) * 4;
+    constexpr int FLAGS = R * SLOT > EPI ? R * SLOT : EPI;  // [BM] row bytes after the tile
+    __shared__ __attribute__((aligned(16))) unsigned char smem[FLAGS + BM];
+    unsigned char *const flags = smem + FLAGS;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    // XCD-aware tile order, N fastest (as the fp32 kernels)
+    const int nb = gridDim.x;
+    const int full = nb & ~7;
+    int lin = blockIdx.x;
+    if (lin < full) {
+        const int per = full >> 3;
+        lin = (lin & 7) * per + (lin >> 3);
+    }
+    const int tm = lin / p.tiles_n;
+    const int tn = lin - tm * p.tiles_n;
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int ks = blockIdx.z;
+    const int kbeg = ks * p.kchunk;
+    const int kend = min(p.K, kbeg + p.kchunk);
+    const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
+    constexpr unsigned OOB = 0x80000000u;  // past every resource's end (extents are < 2^31 bytes)
+
+    // ---- A: this lane's row and its 8 k of each 16 -----------------------------------------
+    const int li = lane & 31;
+    const int lh = lane >> 5;
+    const __amdgpu_buffer_rsrc_t ra =
+        __builtin_amdgcn_make_buffer_rsrc((void *)p.a.p, (short)0, (int)p.a_bytes, 0x00020000);
+    unsigned aoff = OOB, aoff2 = OOB;
+    int aih = -0x40000000, aiw = -0x40000000;  // fails the window bounds test
+    {
+        const int m = m0 + 32 * wave + li;
+        if (m < p.M) {
+            if (AMODE == AM_CAT) {
+                const int n = fdiv(m, p.div_ohw), rr = m - n * p.a2.OH * p.a2.OW;
+                const int oh = fdiv(rr, p.div_ow), ow = rr - oh * p.a2.OW;
+                aoff2 = (unsigned)(((n * p.a2.H + oh * p.a2.SH) * p.a2.W + ow * p.a2.SW) * p.a2.C) * 4u;
+            }
+            if (AMODE == AM_CONV_VEC) {
+                const int n = fdiv(m, p.div_ohw), rr = m - n * p.a.OH * p.a.OW;
+                const int oh = fdiv(rr, p.div_ow), ow = rr - oh * p.a.OW;
+                aih = oh * p.a.SH - p.a.PT;
+                aiw = ow * p.a.SW - p.a.PL;
+                aoff = (unsigned)(((n * p.a.H + aih) * p.a.W + aiw) * p.a.C) * 4u;
+            } else {
+                aoff = (unsigned)m * (unsigned)p.a.rs * 4u;
+            }
+        }
+    }
+    f4 va[2][4];        // [set][16-k block, half of the lane's 8 k]
+    int ka = kbeg;      // the stage the next A loads fetch
+    auto load_a = [&](f4 (&v)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int k = ka + 16 * s + 8 * lh;
+            const bool k0 = k < kend, k1 = k + 4 < kend;
+            if constexpr (AMODE == AM_VEC) {
+                const unsigned o = aoff + (unsigned)k * 4u;
+                v[2 * s] = buf_load4(ra, k0 ? o : OOB);
+                v[2 * s + 1] = buf_load4(ra, k1 ? o + 16u : OOB);
+            } else if constexpr (AMODE == AM_CAT) {
+                // k1 is a multiple of the 32-wide stage, so a whole stage reads one source
+                const bool second = ka >= p.k1;
+                const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+                    (void *)(second ? p.a2.p : p.a.p), (short)0, (int)(second ? p.a2_bytes : p.a_bytes), 0x00020000);
+                const unsigned o = second ? aoff2 + (unsigned)(k - p.k1) * 4u : aoff + (unsigned)k * 4u;
+                v[2 * s] = buf_load4(r, k0 ? o : OOB);
+                v[2 * s + 1] = buf_load4(r, k1 ? o + 16u : OOB);
+            } else {  // cg % 8 == 0: the 8 k share a tap
+                const int t = fdiv(k, p.div_cg), kh = fdiv(t, p.div_kw);
+                const int dh = kh * p.a.DH, dw = (t - kh * p.a.KW) * p.a.DW;
+                const bool ok = k0 && (unsigned)(aih + dh) < (unsigned)p.a.H && (unsigned)(aiw + dw) < (unsigned)p.a.W;
+                const unsigned o =
+                    ok ? aoff + (unsigned)((dh * p.a.W + dw) * p.a.C + (k - t * p.a.cg)) * 4u : OOB;
+                v[2 * s] = buf_load4(ra, o);
+                v[2 * s + 1] = buf_load4(ra, o + 16u);
+            }
+        }
+        ka += BK;
+    };
+    unsigned seen = 0;  // magnitude bits of the row's leading parts (see below)
+    auto split_a = [&](const f4 &x, const f4 &y, bf8 (&a)[3]) __attribute__((always_inline)) {
+        uint4_t h, m, l;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const f4 &v = e < 2 ? x : y;
+            unsigned u0, u1, u2;
+            split3(v[2 * (e & 1)], v[2 * (e & 1) + 1], u0, u1, u2);
+            h[e] = u0;
+            m[e] = u1;
+            l[e] = u2;
+        }
+        seen |= (h[0] | h[1]) | (h[2] | h[3]);
+        a[0] = __builtin_bit_cast(bf8, h);
+        a[1] = __builtin_bit_cast(bf8, m);
+        a[2] = __builtin_bit_cast(bf8, l);
+    };
+
+    // ---- B: 1 KB copy c of a stage is plane c % 3 of 16-k block c / 3 % 2 of column block c / 6 ----
+    const __amdgpu_buffer_rsrc_t rb =
+        __builtin_amdgcn_make_buffer_rsrc((void *)planes, (short)0, (int)plane_bytes, 0x00020000);
+    const unsigned nb_bytes = (unsigned)kblocks * 3072u;
+    static_assert(6 % DMA == 0, "a wave's copies lie in one column block");
+    const int block = n0 / 32 + wave * DMA / 6;
+    // column blocks past N lie past the resource's end, whatever stage is added
+    unsigned boff = block * 32 < p.N
+                        ? (unsigned)block * nb_bytes + (unsigned)(kbeg >> 4) * 3072u +
+                              (unsigned)(wave * DMA % 6) * 1024u + (unsigned)lane * 16u
+                        : OOB;
+    auto copy_b = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < DMA; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void *)(smem + slot * SLOT + (wave * DMA + i) * 1024), 16,
+                                                     (int)boff, i * 1024, 0, 0);
+        boff += 6144u;
+    };
+
+    floatx16 acc[RN], cor[RN];
+#pragma unroll
+    for (int j = 0; j < RN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[j][r] = cor[j][r] = 0.0f;
+
+    // One 16-k step: multiply fragments a by the step's B while the next step's A (x, y) is split
+    // into `next`.
+    auto step = [&](const bf8 (&a)[3], const unsigned char *bs, const f4 &x, const f4 &y, bf8 (&next)[3])
+                    __attribute__((always_inline)) {
+        constexpr int G = RN < 2 ? RN : 2;  // column blocks at a time: independent chains, few registers
+        split_a(x, y, next);
+#pragma unroll
+        for (int j0 = 0; j0 < RN; j0 += G) {
+            bf8 b[G][3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+#pragma unroll
+                for (int j = 0; j < G; ++j)
+                    b[j][q] = *reinterpret_cast<const bf8 *>(bs + (j0 + j) * 6144 + q * 1024 + lane * 16);
+#define MGC_MFMA(C, QA, QB)                          \
+    _Pragma("unroll") for (int j = 0; j < G; ++j)    \
+        C[j0 + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[QA], b[j][QB], C[j0 + j], 0, 0, 0);
+            MGC_MFMA(acc, 0, 0)
+            MGC_MFMA(cor, 2, 0)
+            MGC_MFMA(cor, 1, 0)
+            MGC_MFMA(cor, 1, 1)
+            MGC_MFMA(cor, 0, 1)
+            MGC_MFMA(cor, 0, 2)
+#undef MGC_MFMA
+        }
+    };
+    // Stage kt: its copies and A loads have landed once at most the next stage's are outstanding
+    // (R = 3), and every wave has read the slot that the new copies overwrite. Loads past the
+    // end are masked, so the loop needs no tests.
+    int slot = 0;
+    bf8 a0[3], a1[3];
+    auto stage = [&](f4 (&v)[4], f4 (&w)[4]) __attribute__((always_inline)) {
+        barrier_stage<(R - 2) * (DMA + 4)>();
+        copy_b(slot == 0 ? R - 1 : slot - 1);
+        const unsigned char *const bs = smem + slot * SLOT;
+        step(a0, bs, v[2], v[3], a1);
+        load_a(v);
+        step(a1, bs + 3072, w[0], w[1], a0);
+        slot = slot == R - 1 ? 0 : slot + 1;
+    };
+
+    for (int i = tid; i < BM / 4; i += 64 * WAVES) reinterpret_cast<unsigned *>(flags)[i] = 0;
+    static_assert(R == 3, "the waits above count for a ring of three");
+    copy_b(0);
+    load_a(va[0]);
+    asm volatile("" ::: "memory");  // the stages' loads stay in order: the waits count them
+    copy_b(1);
+    load_a(va[1]);
+    asm volatile("" ::: "memory");
+    split_a(va[0][0], va[0][1], a0);
+    for (int kt = nk >> 1; kt > 0; --kt) {
+        stage(va[0], va[1]);
+        stage(va[1], va[0]);
+    }
+    if (nk & 1) stage(va[0], va[1]);
+    wait_vmcnt<0>();  // masked copies past the end may still be writing the ring
+    __syncthreads();
+
+    // A row whose elements (as this lane saw them: a half of its k) are all below 2^-95 and not
+    // all zero: bf16 exponent bits of the OR below 32.
+    if (((seen | (seen >> 16)) & 0x7fffu) - 1u < 0x0fffu) flags[32 * wave + li] = 1;
+    float *const Cs = reinterpret_cast<float *>(smem);
+#pragma unroll
+    for (int j = 0; j < RN; ++j) {
+        acc[j] += cor[j];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            Cs[(32 * wave + (r >> 2) * 8 + lh * 4 + (r & 3)) * (BN + 8) + j * 32 + li] = acc[j][r];
+    }
+    __syncthreads();
+    const unsigned char *const cflags = planes + plane_bytes;
+    const auto fix = [&](f4 &v, int rl, int cl, int ncol) __attribute__((always_inline)) {
+        const float z = (v[0] * 0.0f + v[1] * 0.0f) + (v[2] * 0.0f + v[3] * 0.0f);  // NaN if a sum is not finite
+        const unsigned mark = flags[rl] | *reinterpret_cast<const unsigned *>(cflags + n0 + cl);
+        if (z != z || mark) {
+#pragma unroll 1
+            for (int e = 0; e < ncol; ++e) {
+                const float s = dot_fp32<AMODE>(p, p.a.p, p.b.p, m0 + rl, n0 + cl + e, kbeg, kend);
+                v[0] = e == 0 ? s : v[0];
+                v[1] = e == 1 ? s : v[1];
+                v[2] = e == 2 ? s : v[2];
+                v[3] = e == 3 ? s : v[3];
+            }
+        }
+    };
+    gemm_lds_to_global<BM, BN, decltype(fix), 64 * WAVES>(p, Cs, m0, n0, ks, 0, 0, fix);
+}
+
+template <int RN, int WAVES>
+static SplitKernel pick(int am) {
+    return am == AM_VEC   ? &gemm_split_kernel<RN, WAVES, 3, AM_VEC>
+           : am == AM_CAT ? &gemm_split_kernel<RN, WAVES, 3, AM_CAT>
+                          : &gemm_split_kernel<RN, WAVES, 3, AM_CONV_VEC>;
+}
+
+SplitKernel pick_split(int am, int bn) { return bn == 128 ? pick<4, 4>(am) : pick<2, 4>(am); }
+
+}  // namespace mgc

@@ -252,6 +252,22 @@ int mgc_hip_model_init(mgc_hip_model *m, const unsigned char *weights_host, unsi
     return MGC_OK;
 }
 
+int mgc_hip_model_init_planes(mgc_hip_model *m, const unsigned char *weights_host, unsigned char **A,
+                              unsigned char **W, const mgc_hip_planes_entry *planes, int n_planes) {
+    const bool fresh = m && !m->state;
+    const int rc = mgc_hip_model_init(m, weights_host, A, W);
+    if (rc != MGC_OK || !fresh) return rc;
+    ModelState *s = state(m);
+    s->exec.launch_error = 0;
+    for (int i = 0; i < n_planes; ++i)
+        mgc_hip_gemm_make_planes(&s->exec, reinterpret_cast<const float *>(s->W + planes[i].weights_off), planes[i].k,
+                                 planes[i].n, planes[i].k, s->A + planes[i].arena_off);
+    hipError_t err = s->exec.launch_error ? (hipError_t)s->exec.launch_error : hipStreamSynchronize(s->stream);
+    if (err == hipSuccess) return MGC_OK;
+    mgc_hip_model_release(m);
+    return fail("weight planes", err);
+}
+
 static int check_ptrs(mgc_hip_model *m, unsigned char *A, const unsigned char *W) {
     if (!m || !m->state) return MGC_ERR_ARGS;
     ModelState *s = state(m);

@@ -111,6 +111,9 @@ def load_kernel_library() -> ctypes.CDLL:
         lib.mgc_hip_gemm_workspace.argtypes = [ctypes.c_int] * 4
         lib.mgc_hip_gemm_layer_norm_workspace.restype = ctypes.c_long
         lib.mgc_hip_gemm_layer_norm_workspace.argtypes = [ctypes.c_int] * 3
+        for fn in (lib.mgc_hip_gemm_planes_bytes, lib.mgc_hip_gemm_planes_workspace):
+            fn.restype = ctypes.c_long
+            fn.argtypes = [ctypes.c_int] * 3
         lib.mgc_hip_last_error.restype = ctypes.c_char_p
         lib.mgc_hip_version.restype = ctypes.c_char_p
         lib.mgc_hip_device_count.restype = ctypes.c_int
@@ -119,8 +122,17 @@ def load_kernel_library() -> ctypes.CDLL:
 
 
 def gemm_workspace_floats(m: int, n: int, k: int, batch: int) -> int:
-    """Workspace the kernel library wants for one GEMM (asked at compile time)."""
-    return int(load_kernel_library().mgc_hip_gemm_workspace(m, n, k, batch))
+    """Workspace the kernel library wants for one GEMM (asked at compile time), by its fp32 kernels
+    or, with its right-hand side as planes, by the bf16-split ones."""
+    lib = load_kernel_library()
+    planes = int(lib.mgc_hip_gemm_planes_workspace(m, n, k)) if batch == 1 else 0
+    return max(int(lib.mgc_hip_gemm_workspace(m, n, k, batch)), planes)
+
+
+def gemm_planes_bytes(m: int, n: int, k: int) -> int:
+    """Device bytes of the bf16 planes of a constant k x n right-hand side whose GEMM over m rows the
+    kernel library runs on the bf16 matrix cores (0: it keeps the fp32 kernels)."""
+    return int(load_kernel_library().mgc_hip_gemm_planes_bytes(m, n, k))
 
 
 def gemm_layer_norm_workspace_floats(m: int, n: int, k: int) -> int:

@@ -639,6 +639,7 @@ class HipEmitter:
         profile: bool = False,
         gemm_workspace: Callable[[int, int, int, int], int] | None = None,
         gemm_ln_workspace: Callable[[int, int, int], int] | None = None,
+        gemm_planes: Callable[[int, int, int], int] | None = None,
     ) -> None:
         unsupported = sorted({n.op for n in graph.nodes} - self.SUPPORTED)
         if unsupported:
@@ -649,6 +650,11 @@ class HipEmitter:
         self.graph = graph
         self.profile = profile
         self._gemm_ws = gemm_workspace
+        # Right-hand sides laid out as bf16 planes at init: (weights offset, n, k) -> the planes'
+        # offset within the region past the scratch area, and that region's bytes.
+        self._gemm_planes = gemm_planes
+        self._planes: dict[tuple[int, int, int], int] = {}
+        self._planes_bytes = 0
         # id(last 1 x 1 conv) -> its projection shortcut, and the shortcuts' ids. The shortcut's
         # input is then read at the last conv's step, which the plan must keep it alive for.
         self._shortcut: dict[int, Node] = find_projection_shortcuts(graph) if FUSE_PROJECTION_SHORTCUT else {}
@@ -703,6 +709,7 @@ class HipEmitter:
         self.plan = plan_memory(graph, strategy=strategy, alignment=ALIGN, inplace=inplace,
                                 workspace=self._workspace_bytes, extra_reads=keep)
         self.weights = WeightsBuilder()
+        self._packed_off: dict[str, int] = {}  # operand text of a packed right-hand side -> weights offset
         self.body: list[str] = []
         self.kernels: dict[str, int] = {}
         self._gemm_flops = 0
@@ -1406,9 +1413,15 @@ class HipEmitter:
                 parts.append(f"g.batch_dims[{d}] = {dim}; g.a_bs[{d}] = {abs_}L; g.b_bs[{d}] = {bbs}L; g.c_bs[{d}] = {cbs}L; g.r_bs[{d}] = {rbs}L;")
         parts.append(f"g.workspace = {workspace}; g.workspace_floats = {workspace_floats}L;")
         parts += extra
+        planes = self._planes_ptr(m, n, k, b) if not batch and depthwise is None and mbconv is None else None
         if layer_norm is not None:
             scale, lbias, eps, out = layer_norm
-            parts.append(f"mgc_hip_gemm_layer_norm(x, &g, {scale}, {lbias}, {eps}, {out});")
+            if planes is not None:
+                parts.append(f"mgc_hip_gemm_planes_layer_norm(x, &g, {planes}, {scale}, {lbias}, {eps}, {out});")
+            else:
+                parts.append(f"mgc_hip_gemm_layer_norm(x, &g, {scale}, {lbias}, {eps}, {out});")
+        elif planes is not None:
+            parts.append(f"mgc_hip_gemm_planes(x, &g, {planes});")
         elif depthwise is not None:
             parts += [depthwise, "mgc_hip_gemm_dw(x, &g, &d);"]
         elif mbconv is not None and stem is not None:
@@ -1431,7 +1444,30 @@ class HipEmitter:
         """Constant K x N right-hand side stored [N][K]: element (k, n) at n * K + k."""
         k = matrix.shape[0]
         off = self.weights.add(pack_b_nk(matrix), key=key)
-        return self._strided("b", f"(W + {off})", 1, k)
+        spec = self._strided("b", f"(W + {off})", 1, k)
+        self._packed_off[spec[0]] = off
+        return spec
+
+    def _planes_ptr(self, m: int, n: int, k: int, b: list[str]) -> str | None:
+        """The planes of a packed constant right-hand side, laid out once at init from the weights
+        blob, or None when the library keeps this GEMM on its fp32 kernels. GEMMs that share a
+        matrix share its planes."""
+        off = self._packed_off.get(b[0]) if len(b) == 1 else None
+        if off is None or self._gemm_planes is None:
+            return None
+        nbytes = int(self._gemm_planes(m, n, k))
+        if nbytes <= 0:
+            return None
+        at = self._planes.get((off, n, k))
+        if at is None:
+            at = self._planes[(off, n, k)] = self._planes_bytes
+            self._planes_bytes += (nbytes + ALIGN - 1) // ALIGN * ALIGN
+        return f"(A + {self._planes_off + at})"
+
+    @property
+    def _planes_off(self) -> int:
+        """Start of the planes: past the scratch area, whose size is known before any node is emitted."""
+        return self._scratch_off + (self._scratch_bytes + ALIGN - 1) // ALIGN * ALIGN
 
     def _act(self, node: Node) -> tuple[str, float, float]:
         return (str(node.attrs.get("activation", "none")), float(node.attrs.get("clip_min", 0.0)),
@@ -2189,8 +2225,8 @@ class HipEmitter:
             t = value.tensor_type
             self.copy((t.nbytes,), f"((unsigned char *)out[{j}])", [1], 0, self.ptr(value), [1], 0, 1)
         arena = max(self.plan.arena_bytes, ALIGN)
-        if self._scratch_bytes:
-            arena = self._scratch_off + (self._scratch_bytes + ALIGN - 1) // ALIGN * ALIGN
+        if self._scratch_bytes or self._planes_bytes:
+            arena = self._planes_off + self._planes_bytes
         weights = self.weights
         n_in, n_out = len(self.graph.inputs), len(self.graph.named_outputs())
         in_bytes = ", ".join(f"{v.tensor_type.nbytes}UL" for v in self.graph.inputs) or "0UL"
@@ -2223,7 +2259,7 @@ class HipEmitter:
             f"size_t mgc_arena_bytes(void) {{ return {arena}UL; }}",
             f"size_t mgc_weights_bytes(void) {{ return {weights.nbytes}UL; }}",
             "int mgc_hip_init(const unsigned char *w, unsigned char **A, unsigned char **W) {",
-            "    return mgc_hip_model_init(&MODEL, w, A, W);",
+            *self._init_body(),
             "}",
             "int mgc_run(const void *const *inputs, void *const *outputs, unsigned char *A, const unsigned char *W) {",
             "    return mgc_hip_model_run(&MODEL, inputs, outputs, A, W);",
@@ -2266,6 +2302,15 @@ class HipEmitter:
             node_flops=self._node_flops(),
             gemm_flops=self._gemm_flops,
         )
+
+    def _init_body(self) -> list[str]:
+        if not self._planes:
+            return ["    return mgc_hip_model_init(&MODEL, w, A, W);"]
+        rows = ", ".join(f"{{{off}UL, {self._planes_off + at}UL, {n}, {k}}}" for (off, n, k), at in self._planes.items())
+        return [
+            f"    static const mgc_hip_planes_entry planes[] = {{{rows}}};",
+            f"    return mgc_hip_model_init_planes(&MODEL, w, A, W, planes, {len(self._planes)});",
+        ]
 
     def _node_flops(self) -> list[int]:
         """FLOPs per node, with the nodes a fused attention call absorbs (among them a QKV
@@ -2310,8 +2355,10 @@ def generate_hip(
     profile: bool = False,
     gemm_workspace: Callable[[int, int, int, int], int] | None = None,
     gemm_ln_workspace: Callable[[int, int, int], int] | None = None,
+    gemm_planes: Callable[[int, int, int], int] | None = None,
 ) -> GeneratedModel:
     """Generate the host source and weights blob of a scheduled graph for the hip backend.
     ``gemm_workspace`` / ``gemm_ln_workspace`` ask the kernel library for split-K workspace
-    sizes (without the second, no LayerNorm is fused into a GEMM)."""
-    return HipEmitter(graph, strategy, inplace, profile, gemm_workspace, gemm_ln_workspace).generate()
+    sizes (without the second, no LayerNorm is fused into a GEMM), ``gemm_planes`` which constant
+    right-hand sides it wants as bf16 planes (without it, none)."""
+    return HipEmitter(graph, strategy, inplace, profile, gemm_workspace, gemm_ln_workspace, gemm_planes).generate()

@@ -1,0 +1,45 @@
+"""Constant right-hand sides laid out as bf16 planes: which GEMMs get them and where they lie."""
+
+from __future__ import annotations
+
+import re
+
+from ml_graph_compiler import builders
+from ml_graph_compiler.codegen import build as native
+from ml_graph_compiler.codegen.hip import generate_hip
+from ml_graph_compiler.passes import optimize
+from ml_graph_compiler.schedule import schedule
+
+
+def _generate(graph, planes=True):
+    optimize(graph, "O3")
+    schedule(graph)
+    return generate_hip(graph, gemm_workspace=native.gemm_workspace_floats,
+                        gemm_ln_workspace=native.gemm_layer_norm_workspace_floats,
+                        gemm_planes=native.gemm_planes_bytes if planes else None)
+
+
+def test_large_gemms_read_planes_past_the_plan(hip_cache):
+    make = lambda: builders.transformer(batch=16, seq=128, d_model=256, heads=4, layers=2, vocab=4096, gelu="erf", causal=False)  # noqa: E731
+    plain, gen = _generate(make(), planes=False), _generate(make())
+    assert "planes" not in plain.source and gen.plan.arena_bytes == plain.plan.arena_bytes
+    assert gen.weights.digest() == plain.weights.digest()  # the blob stays as it is
+    rows = [tuple(map(int, r)) for r in re.findall(r"\{(\d+)UL, (\d+)UL, (\d+), (\d+)\}", gen.source)]
+    assert rows and len({r[0] for r in rows}) == len(rows)
+    used = {int(o) for o in re.findall(r"mgc_hip_gemm_planes(?:_layer_norm)?\(x, &g, \(A \+ (\d+)\)", gen.source)}
+    assert used == {at for _, at, _, _ in rows}
+    end = plain.arena_bytes  # the plan and the scratch area
+    for off, at, n, k in sorted(rows, key=lambda r: r[1]):
+        assert at % 256 == 0 and at >= end and off + 4 * n * k <= gen.weights.nbytes
+        end = at + native.gemm_planes_bytes(2048, n, k)
+        assert end - at >= n * k * 6
+    assert end <= gen.arena_bytes
+    native.build_model_library(gen.source, cache_dir=hip_cache, name="planes")
+
+
+def test_small_gemms_keep_the_fp32_kernels():
+    assert "planes" not in _generate(builders.single_gemm()).source
+    assert "planes" not in _generate(builders.mlp()).source
+    for m, n, k in ((1, 50257, 768), (128, 768, 768), (2048, 32, 768), (2048, 768, 32), (0, 1, 1)):
+        assert native.gemm_planes_bytes(m, n, k) == 0
+    assert native.gemm_planes_bytes(2048, 3072, 768) >= 3072 * 768 * 6

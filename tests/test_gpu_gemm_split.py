@@ -1,0 +1,228 @@
+"""fp32 GEMMs on the bf16 matrix cores (mgc_hip_gemm_planes) against float64.
+
+Both tile shapes are pinned through mgc_hip_gemm_args.kernel at the edges of their tiles (128 rows,
+64 or 128 columns, 32 k per stage, 16 k per MFMA), for row-major A, NHWC convolutions and a
+concatenated K, with a K split and a rotating epilogue. The tolerance is the standard bound of a
+summation: with S = sum |a||b| of an element, at most 6 K / 16 + 8 roundings of 2^-24 S for the MFMA
+accumulations and the epilogue, and 2^-23 S for the products the split drops.
+
+Operands the split cannot carry are recomputed in fp32: infinities and NaN come out as float
+arithmetic has them, rows or columns below 2^-95 keep fp32 precision.
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from capi import ACTS, MGC_ERR_ARGS, MGC_OK, MGC_OP_CONV_NHWC, GemmArgs, Hip, bind
+from ml_graph_compiler.codegen.build import load_kernel_library
+from oracle import interpreter as oracle
+
+pytestmark = pytest.mark.gpu
+
+FAMILIES = {"128x128": 8, "128x64": 9}
+
+
+class Runner:
+    def __init__(self) -> None:
+        self.lib = load_kernel_library()
+        bind(self.lib)
+        self.lib.mgc_hip_gemm_make_planes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_long, ctypes.c_int,
+                                                      ctypes.c_int, ctypes.c_void_p]
+        self.lib.mgc_hip_gemm_planes.argtypes = [ctypes.c_void_p] * 3
+        self.hip = Hip()
+        self.x = self.lib.mgc_hip_exec_create(None)
+        assert self.x, self.lib.mgc_hip_last_error()
+
+    def planes(self, b: np.ndarray) -> tuple[int, int]:
+        """Device addresses of b ([N][K]) and of its planes."""
+        n, k = b.shape
+        pb = self.hip.upload(b)
+        planes = self.hip.alloc((n + 31) // 32 * 32 * ((k + 31) // 32 * 32) * 6 + (n + 31) // 32 * 32 + 256)
+        self.lib.mgc_hip_gemm_make_planes(self.x, pb, k, n, k, planes)
+        return pb, planes
+
+    def run(self, g: GemmArgs, planes: int) -> int:
+        self.lib.mgc_hip_gemm_planes(self.x, ctypes.byref(g), planes)
+        return self.lib.mgc_hip_exec_status(self.x)
+
+    def gemm(self, family: str, a: np.ndarray, b: np.ndarray, fill=None, split: int = 1, m: int | None = None,
+             bias=None, bias_mode=0, res=None, alpha=1.0, beta=1.0, act="none", lo=-0.5, hi=0.75) -> np.ndarray:
+        m = a.shape[0] if m is None else m
+        n, k = b.shape
+        g = GemmArgs()
+        g.M, g.N, g.K = m, n, k
+        g.a.p, g.a.rs, g.a.cs = self.hip.upload(a), k, 1
+        g.b.rs, g.b.cs = 1, k
+        g.b.p, planes = self.planes(b)
+        g.c, g.ldc = self.hip.empty(4 * m * n), n
+        g.alpha, g.beta, g.bias_mode = alpha, beta, bias_mode
+        g.bias = self.hip.upload(bias) if bias is not None else None
+        if res is not None:
+            g.res, g.ldr = self.hip.upload(res), n
+        g.act, g.lo, g.hi = ACTS.index(act), lo, hi
+        g.kernel, g.split_k = FAMILIES[family], split
+        if split > 1:
+            g.workspace, g.workspace_floats = self.hip.empty(4 * split * m * n), split * m * n
+        if fill is not None:
+            fill(g)
+        code = self.run(g, planes)
+        assert code == MGC_OK, (code, self.lib.mgc_hip_last_error())
+        out = self.hip.download(g.c, (m, n))
+        self.hip.free()
+        return out
+
+
+@pytest.fixture(scope="module")
+def runner():
+    r = Runner()
+    yield r
+    r.lib.mgc_hip_exec_destroy(r.x)
+
+
+def _bound(a64: np.ndarray, b64: np.ndarray, k: int) -> np.ndarray:
+    s = np.abs(a64) @ np.abs(b64).T
+    return (6 * k / 16 + 10) * 2.0**-24 * s
+
+
+def _check(got, a64, b64, extra=0.0, bias=None, bias_mode=0, res=None, alpha=1.0, beta=1.0, act="none"):
+    y = alpha * (a64 @ b64.T)
+    scale = abs(alpha) * _bound(a64, b64, a64.shape[1])
+    if bias_mode == 1:
+        y = y + bias[None, :].astype(np.float64)
+    if bias_mode == 2:
+        y = y + bias[:, None].astype(np.float64)
+    if res is not None:
+        y = y + beta * res.astype(np.float64)
+    scale = scale + 2.0**-22 * np.abs(y) + 1e-30 + extra  # the epilogue's own roundings
+    if act != "none":
+        y = oracle.activation(y, {"activation": act, "clip_min": -0.5, "clip_max": 0.75})
+        scale = 1.2 * scale + 5e-7  # slope at most 1.13 (GELU), the activations' own approximation
+    assert np.all(np.abs(got - y) <= scale), float(np.max(np.abs(got - y) / scale))
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+@pytest.mark.parametrize("k", [4, 16, 28, 32, 36, 64, 68, 100, 260, 1028])
+def test_shapes(runner, family, k):
+    """Rows and columns at the tiles' edges, K at the stages', every epilogue and K splits."""
+    rng = np.random.default_rng(k)
+    for i, (m, n) in enumerate([(1, 1), (31, 33), (127, 63), (128, 64), (129, 65), (130, 127), (200, 128), (257, 129), (64, 260)]):
+        a = rng.standard_normal((m, k)).astype(np.float32)
+        b = (rng.standard_normal((n, k)) * 0.1).astype(np.float32)
+        mode = i % 3
+        bias = rng.standard_normal((0, n, m)[mode]).astype(np.float32) if mode else None
+        res = rng.standard_normal((m, n)).astype(np.float32) if i % 2 else None
+        ep = {"bias": bias, "bias_mode": mode, "res": res, "alpha": 0.5 if i % 4 == 3 else 1.0, "beta": -0.75, "act": ACTS[(i + k) % 7]}
+        split = (1, 2, 3)[i % 3] if k >= 64 else 1
+        got = runner.gemm(family, a, b, split=split, **ep)
+        _check(got, a.astype(np.float64), b.astype(np.float64), **ep)
+
+
+def _im2col(x: np.ndarray, kh: int, stride: int, pad: int) -> np.ndarray:
+    n, h, w, c = x.shape
+    xp = np.pad(x, ((0, 0), (pad, pad), (pad, pad), (0, 0)))
+    oh, ow = (h + 2 * pad - kh) // stride + 1, (w + 2 * pad - kh) // stride + 1
+    cols = [xp[:, i : i + stride * (oh - 1) + 1 : stride, j : j + stride * (ow - 1) + 1 : stride] for i in range(kh) for j in range(kh)]
+    return np.stack(cols, 3).reshape(n * oh * ow, kh * kh * c)
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+@pytest.mark.parametrize("c,kh,stride,pad,hw", [(8, 3, 1, 1, 9), (8, 3, 2, 0, 15), (24, 3, 1, 1, 7), (64, 3, 1, 1, 12), (64, 1, 2, 0, 14), (40, 5, 2, 2, 11)])
+def test_convolutions(runner, family, c, kh, stride, pad, hw):
+    rng = np.random.default_rng(c + kh)
+    x = rng.standard_normal((3, hw, hw, c)).astype(np.float32)
+    cols = _im2col(x, kh, stride, pad)
+    m, k = cols.shape
+    n = 70
+    b = (rng.standard_normal((n, k)) * 0.1).astype(np.float32)
+    o = (hw + 2 * pad - kh) // stride + 1
+
+    def fill(g):
+        g.a.kind, g.a.p = MGC_OP_CONV_NHWC, runner.hip.upload(x)
+        g.a.H = g.a.W = hw
+        g.a.C = g.a.cg = c
+        g.a.KH = g.a.KW = kh
+        g.a.SH = g.a.SW = stride
+        g.a.DH = g.a.DW = 1
+        g.a.PT = g.a.PL = pad
+        g.a.OH = g.a.OW = o
+
+    got = runner.gemm(family, x, b, fill=fill, m=m, act="relu")
+    _check(got, cols.astype(np.float64), b.astype(np.float64), act="relu")
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+def test_concatenated_k(runner, family):
+    """Columns past k1 come from an image sampled at a stride (a projection shortcut)."""
+    rng = np.random.default_rng(5)
+    nb, hw, c2, k1, n = 2, 9, 36, 64, 100
+    o = (hw + 1) // 2
+    x = rng.standard_normal((nb, hw, hw, c2)).astype(np.float32)
+    a = rng.standard_normal((nb * o * o, k1)).astype(np.float32)
+    whole = np.concatenate([a, x[:, ::2, ::2].reshape(-1, c2)], axis=1)
+    b = (rng.standard_normal((n, k1 + c2)) * 0.1).astype(np.float32)
+
+    def fill(g):
+        g.a.rs, g.k1 = k1, k1
+        g.a2.kind, g.a2.p = MGC_OP_CONV_NHWC, runner.hip.upload(x)
+        g.a2.H = g.a2.W = hw
+        g.a2.C = g.a2.cg = c2
+        g.a2.KH = g.a2.KW = g.a2.DH = g.a2.DW = 1
+        g.a2.SH = g.a2.SW = 2
+        g.a2.OH = g.a2.OW = o
+
+    got = runner.gemm(family, a, b, fill=fill)
+    _check(got, whole.astype(np.float64), b.astype(np.float64))
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+def test_values_the_split_cannot_carry(runner, family):
+    """Infinities, NaN, overflow and the largest floats as fp32 has them; tiny rows and columns to
+    fp32 precision; zeros exact; everything else in the same tiles untouched."""
+    rng = np.random.default_rng(9)
+    m, n, k = 140, 72, 96
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.choice([0.5, -2.0, 1.0, 0.25, -1.5], (n, k)).astype(np.float32)  # exact in bf16: zero low parts
+    a[3, 5] = np.inf
+    a[4, 6] = -np.inf
+    a[5, 7] = np.nan
+    a[6, 8], a[6, 9] = np.inf, -np.inf
+    a[7, 10] = 3.4e38
+    a[8] = 0.0
+    a[9] *= np.float32(2.0**-120)
+    a[130] *= np.float32(2.0**-100)
+    b[11, 3] = np.inf
+    b[12] *= np.float32(2.0**-118)
+    got = runner.gemm(family, a, b)
+    with np.errstate(all="ignore"):
+        # small whole steps of the exact sum, then rounded to float: infinities and NaN as float has them
+        want = (a.astype(np.float64) @ b.astype(np.float64).T).astype(np.float32)
+        bound = _bound(np.where(np.isfinite(a), a, 0).astype(np.float64), np.where(np.isfinite(b), b, 0).astype(np.float64), k)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isposinf(got), np.isposinf(want))
+    np.testing.assert_array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= 4 * bound[ok] + 2.0**-148)
+    assert np.all(got[8][np.isfinite(b).all(1)] == 0.0)
+
+
+def test_refusals(runner):
+    """The families need planes and an A they can read; mgc_hip_gemm has none."""
+    a, b = np.ones((128, 32), np.float32), np.ones((64, 32), np.float32)
+    g = GemmArgs()
+    g.M, g.N, g.K, g.alpha = 128, 64, 32, 1.0
+    g.a.p, g.a.rs, g.a.cs = runner.hip.upload(a), 32, 1
+    g.b.rs, g.b.cs = 1, 32
+    g.b.p, planes = runner.planes(b)
+    g.c, g.ldc, g.kernel = runner.hip.empty(4 * 128 * 64), 64, 9
+    runner.lib.mgc_hip_gemm(runner.x, ctypes.byref(g))
+    assert runner.lib.mgc_hip_exec_status(runner.x) == MGC_ERR_ARGS
+    g.a.p = g.a.p + 4  # not 16-byte aligned: refused when pinned, fp32 kernels otherwise
+    g.M = 127
+    assert runner.run(g, planes) == MGC_ERR_ARGS
+    g.kernel = 0
+    assert runner.run(g, planes) == MGC_OK
+    runner.hip.free()
