@@ -618,11 +618,11 @@ typedef struct {
 
 int mgc_hip_model_init_planes(mgc_hip_model *m, const unsigned char *weights_host, unsigned char **A,
                               unsigned char **W, const mgc_hip_planes_entry *planes, int n_planes);
-/* Host inputs/outputs: H2D copy, replay of the captured hipGraph, D2H copy, synchronize. */
+/* Host inputs/outputs: H2D copy, the forward (a long one as a replayed hipGraph), D2H copy, synchronize. */
 int mgc_hip_model_run(mgc_hip_model *m, const void *const *inputs, void *const *outputs,
                       unsigned char *A, const unsigned char *W);
-/* Device inputs/outputs (for example torch tensors); the graph is re-captured when the pointer
- * set changes. Synchronizes and returns the status. */
+/* Device inputs/outputs (for example torch tensors); a long forward is captured when a
+ * set of pointers comes a second time in a row. Synchronizes and returns the status. */
 int mgc_hip_model_run_device(mgc_hip_model *m, const void *const *inputs, void *const *outputs,
                              unsigned char *A, const unsigned char *W);
 /* Resident-input execution for benchmarks: upload once, then enqueue replays without copies. */
@@ -635,7 +635,7 @@ int mgc_hip_model_download(mgc_hip_model *m, void *const *outputs);
 int mgc_hip_model_profile_run(mgc_hip_model *m, int replays);
 const double *mgc_hip_model_profile_data(mgc_hip_model *m);
 void mgc_hip_model_profile_reset(mgc_hip_model *m);
-/* Time `replays` graph replays between two hipEvents on the model stream; milliseconds. */
+/* Time `replays` forwards between two hipEvents on the model stream; milliseconds. */
 double mgc_hip_model_time_graph(mgc_hip_model *m, int replays);
 void mgc_hip_model_release(mgc_hip_model *m);
 

@@ -60,7 +60,7 @@ int mgc_hip_init(const unsigned char *weights_host, unsigned char **A, unsigned 
 int mgc_run_device(const void *const *inputs, void *const *outputs, unsigned char *A,
                    const unsigned char *W);
 
-/* Benchmark support: stage host inputs once, enqueue `replays` hipGraph replays, wait. */
+/* Benchmark support: stage host inputs once, enqueue `replays` forwards, wait. */
 int mgc_hip_upload(const void *const *inputs);
 int mgc_hip_launch(int replays);
 int mgc_hip_sync(void);

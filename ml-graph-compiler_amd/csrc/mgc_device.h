@@ -9,12 +9,13 @@
 // One model's execution context (opaque to generated code).
 struct mgc_hip_exec {
     hipStream_t stream;
-    int *flag;          // device int: 1 after an out-of-range Gather index
+    int *flag;          // int that kernels write: 1 after an out-of-range Gather index
     int profiling;      // 1 while an eager profiled pass runs
     int n_nodes;
     hipEvent_t *ev_begin;
     hipEvent_t *ev_end;
     int launch_error;   // first launch failure seen since the last check (hipError_t)
+    int launches;       // kernels launched since the runtime last cleared it
 };
 
 namespace mgc {

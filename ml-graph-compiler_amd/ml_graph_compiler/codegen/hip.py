@@ -4,7 +4,7 @@ The emitter walks the scheduled graph once and writes one C++ translation unit o
 a forward function with one libmgc_hip.so launcher call per node, every arena, weights, input
 and output pointer a constant offset, plus the exports of include/mgc_model.h. Device work is
 all in the prebuilt kernel library (hand-written gfx950 kernels), so a model builds with g++ in
-about a second and the runtime captures the forward into a hipGraph on first use.
+about a second and the runtime replays a long forward as a captured hipGraph.
 
 Lowering per operator family:
 

@@ -5,9 +5,9 @@ profile, save/load, the thread and blocking knobs, report) so that callers switc
 passing ``backend="hip"``. Differences that follow from the device:
 
 * mgc_hip_init allocates the model's single HBM block and uploads the weights once; ``run``
-  stages host inputs into it, replays the captured hipGraph and copies the outputs back.
+  stages host inputs into it, runs the forward (a long one as a hipGraph) and copies the outputs back.
 * ``run_device`` takes device pointers (for example torch tensors' data_ptr) and skips the copies;
-  ``benchmark_device`` times graph replays on resident inputs with hipEvents.
+  ``benchmark_device`` times forwards on resident inputs with hipEvents.
 * ``profile`` returns per-node seconds measured by hipEvent pairs in eager replays.
 * A missing GPU or HIP failure raises CodegenError; an out-of-range Gather raises GraphError.
 """
@@ -62,7 +62,7 @@ def _aligned_copy(weights: np.ndarray, alignment: int = 256) -> np.ndarray:
 class HipCompiledModel:
     """A model compiled for MI355X: ``run(feeds)`` returns outputs as numpy arrays.
 
-    Calls are serialized with a lock because they share the model's arena and hipGraph."""
+    Calls are serialized with a lock because they share the model's arena and hipGraphs."""
 
     backend = "hip"
 
@@ -205,7 +205,7 @@ class HipCompiledModel:
         self._check(code, "mgc_hip_upload")
 
     def launch(self, replays: int = 1) -> None:
-        """Enqueue graph replays on the staged inputs without waiting."""
+        """Enqueue forwards on the staged inputs without waiting."""
         with self._lock:
             self._check(self.lib.mgc_hip_launch(int(replays)), "mgc_hip_launch")
 
@@ -225,7 +225,7 @@ class HipCompiledModel:
         return results
 
     def benchmark_device(self, feeds: Mapping[str, np.ndarray], warmup: int = 3, replays: int = 20) -> float:
-        """Milliseconds per forward: ``replays`` graph replays on resident inputs between two
+        """Milliseconds per forward: ``replays`` of them on resident inputs between two
         hipEvents on the model stream (no host copies inside the timed region)."""
         self.upload(feeds)
         self.launch(warmup)
