@@ -174,7 +174,9 @@ enum {
     MGC_GEMM_REGISTER = 7, /* register-staged operands: every operand form (gemm_mfma_kernel) */
     /* mgc_hip_gemm_planes only: fp32 products on the bf16 matrix cores (gemm_split_kernel), by tile */
     MGC_GEMM_SPLIT_128X128 = 8,
-    MGC_GEMM_SPLIT_128X64 = 9
+    MGC_GEMM_SPLIT_128X64 = 9,
+    MGC_GEMM_SPLIT_32X64 = 10, /* K dealt to eight waves (gemm_split_small_kernel) */
+    MGC_GEMM_SPLIT_32X32 = 11
 };
 
 void mgc_hip_gemm(mgc_hip_exec *x, const mgc_hip_gemm_args *g);

@@ -2718,41 +2718,68 @@ static int wave_split_ln(int M, int N, int K, int split) {
 }
 
 // Tile and K split of a GEMM with planes of B (gemm_split.hip), or bm 0 where the fp32 kernels are
-// faster. A launch takes as long as its busiest CU, so a tile shape costs ceil(tiles / 256) times
-// one tile; measured per 32-wide stage, a 128 x 128 tile takes 1.8 times a 128 x 64 one (4096 x 3072
-// x 768: 768 tiles 106 us, 1536 tiles 118 us; 25088 x 128 x 1152: 196 tiles 51 us, 392 tiles 53 us).
-// K is split in up to four where the tiles leave CUs idle, at least 256 k a part (more parts were
-// never faster than the fp32 kernels: 256 x 768 x 3072 in eight 20.0 against 20.7 us), and `split` > 0
-// fixes it.
+// faster: the cheapest of the shapes that can win, by a model of their times. A launch takes as
+// long as its busiest CU, so a tile costs its stages (32 k each) times ceil(workgroups / 256). In
+// microseconds, fitted to the shapes below: 128 x 64 tiles 7 + 0.74 a stage, 128 x 128 tiles
+// 10 + 1.33 a stage, 32 x 64 tiles (K dealt to eight waves) 3 + 2 a round + 0.22 a stage, 32 x 32 tiles the
+// same with 0.19.
 //
-// The fp32 kernels stay where a launch cannot fill the chip: these tiles are large and a stage is
-// a long chain (load, split, multiply), so they win from three quarters of a round of workgroups
-// on (us, fp32 / split: 2048 x 768 x 768, 192 tiles, 25.5 / 23.7; 512 x 2304 x 768, 144 tiles, 23.5 /
-// 24.1; 1024 x 2304 x 768, 288 tiles, 34.7 / 39.3) and with K of 192 on, or from about 1536 tiles
-// on with shorter K (100352 x 256 x 64 46.4 / 40.3; 100352 x 64 x 64, 784 tiles, 16.5 / 17.8; 4096 x 512
-// x 128, 256 tiles, 9.9 / 11.0).
+// 128-row tiles need three quarters of a round of workgroups, evenly filled, and K of 192 on or
+// about six rounds (us, fp32 kernel / this: 2048 x 768 x 768, 192 tiles, 25.5 / 23.7; 25088 x 128 x 1152
+// 67.5 / 50.9; 4096 x 3072 x 768 166 / 106; 512 x 2304 x 768, 144 tiles, 23.5 / 24.1; 1024 x 2304 x 768,
+// 288 tiles, 34.7 / 39.3; 100352 x 256 x 64 46.4 / 40.3; 100352 x 64 x 64, 784 tiles, 16.5 / 17.8). K is split
+// in up to four parts of at least 512 where the tiles leave CUs idle (1568 x 512 x 4608 in four 70.2 /
+// 55.1; parts of 256: 6272 x 128 x 512 13.8 / 17.3); `split` > 0 fixes it (a LayerNorm tail). Over very
+// many columns the planes' bytes bound the launch and padded rows cost nothing (64 x 50257 x 768
+// 92.0 / 57.9).
+// 32 x 64 tiles win from 144 workgroups on while they fill one round (128 x 2304 x 768 11.6 / 10.1, 392 x
+// 1024 x 768 11.7 / 10.3, 3136 x 128 x 1152 15.6 / 12.0), or two with long K (6272 x 128 x 1152 28.2 / 22.1;
+// 1568 x 512 x 1024 23.0 / 24.0); 32 x 32 tiles from 192 on with K of 256 to 384 (196 x 1024 x 256 6.6 / 5.7;
+// 1568 x 128 x 512 6.2 / 6.6), and for a few rows over more columns than the 16 x 16 fp32 tiles take
+// (1 x 50257 x 768 94.3 / 39.0, 32 x 20000 x 768 41.5 / 20.7; 32 x 8000 x 1024 9.2 / 11.0).
+//
+// K not a multiple of four leaves only the element-by-element fp32 kernel (a `loose` A), which these
+// beat everywhere measured (1003 x 1021 x 515 28.5 / 22.3, 33 x 333 x 1021 21.8 / 8.9, 4095 x 3001 x 2047
+// 737 / 325, 7 x 2999 x 77 8.3 / 4.6); its 128 x 128 tiles take 1.8 us a stage, its 32-row tiles are 32 x 32.
 static SplitChoice split_choice(int M, int N, int K, long workspace_floats, int split) {
-    const SplitChoice none{0, 0, 0};
-    if (N < 64 || K < 64 || (N + 63) / 64 * 64 > N + N / 4 || (M + 127) / 128 * 128 > M + M / 3) return none;  // padding
-    SplitChoice best = none;
+    SplitChoice best{0, 0, 0};
+    const bool loose = K % 4 != 0;
+    if (K < 64 || N < 32) return best;
+    auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    auto rounds = [&](long wgs) { return (wgs + kCUs - 1) / kCUs; };
     double best_cost = 0.0;
+    auto take = [&](int bm, int bn, int s, double cost) {
+        if (best.bm && cost >= best_cost) return;
+        best = SplitChoice{bm, bn, s};
+        best_cost = cost;
+    };
     const int stages = (K + 31) / 32;
-    const int max_split = split > 0 ? split : K / 256 < 4 ? (K / 256 > 1 ? K / 256 : 1) : 4;
-    for (int bn = 64; bn <= 128; bn += 64) {
-        const long tiles = (long)((M + 127) / 128) * ((N + bn - 1) / bn);
+    const bool pad32 = (N + 31) / 32 * 32 > N + N / 4, pad64 = (N + 63) / 64 * 64 > N + N / 4;  // columns of padding
+    const bool rows = (M + 127) / 128 * 128 <= M + M / 3 || (M > 32 && N >= 16384);
+    const int max_split = split > 0 ? split : K / 512 < 4 ? (K / 512 > 1 ? K / 512 : 1) : 4;
+    for (int bn = 64; bn <= 128 && (loose || (rows && !pad64)); bn += 64) {
+        const long t = tiles(128, bn);
         for (int s = split > 0 ? split : 1; s <= max_split; ++s) {
-            if (s > 1 && split <= 0 && (tiles >= kCUs || (long)s * M * N > workspace_floats)) break;
-            const long wgs = tiles * s, rounds = (wgs + kCUs - 1) / kCUs;
-            if (wgs < kCUs * 3 / 4 || wgs * 10 < rounds * kCUs * 6 || (K < 192 && wgs < 6 * kCUs)) continue;
-            // microseconds: the stages, and a reduction's launch and traffic
-            double cost = (double)rounds * ((stages + s - 1) / s) * (bn == 128 ? 1.33 : 0.74);
-            if (s > 1) cost += 4.0 + (2.0 * s + 1.0) * M * N * 1e-6;
-            if (!best.bm || cost < best_cost) {
-                best = SplitChoice{128, bn, s};
-                best_cost = cost;
-            }
+            if (s > 1 && split <= 0 && (t >= kCUs || (long)s * M * N > workspace_floats)) break;
+            const long wgs = t * s, r = rounds(wgs);
+            if (!loose && (wgs < kCUs * 3 / 4 || wgs * 10 < r * kCUs * 6 || (K < 192 && wgs < 6 * kCUs))) continue;
+            double cost = (bn == 64 ? 7.0 : 10.0) +
+                          (double)r * ((stages + s - 1) / s) * (bn == 64 ? 0.74 : loose ? 1.8 : 1.33);
+            if (s > 1) cost += 4.0 + (2.0 * s + 1.0) * M * N * 1e-6;  // the reduction's launch and traffic
+            take(128, bn, s, cost);
         }
     }
+    if (split > 0) return best;
+    const long t64 = tiles(32, 64), t32 = tiles(32, 32);
+    const double cost32 = 3.0 + (double)rounds(t32) * (2.0 + 0.19 * stages);
+    if (loose) {
+        take(32, 32, 1, cost32);
+        return best;
+    }
+    if (!pad64 && K >= 128 && t64 >= 144 && (t64 <= kCUs || (t64 <= 2 * kCUs && K > 1024)))
+        take(32, 64, 1, 3.0 + (double)rounds(t64) * (2.0 + 0.22 * stages));
+    if (!pad32 && K >= 256 && K <= 384 && t32 >= 192 && t32 <= kCUs) take(32, 32, 1, cost32);
+    if (!best.bm && M <= 32 && N > 8192) take(32, 32, 1, cost32);
     return best;
 }
 
@@ -3329,17 +3356,22 @@ static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTai
     }
 
     // The bf16-split kernels read eight k of one window tap at a time and B as planes.
-    const bool split_ok = planes != nullptr && dma_ok && batch == 1 && (am != AM_CONV_VEC || p.a.cg % 8 == 0) &&
-                          plane_data_bytes(p.N, p.K) < kMaxRes;
+    // A row-major A need only be 4-byte aligned (at least four columns).
+    const bool loose = am == AM_GEN && nonneg && p.a.kind == MGC_OP_STRIDED && p.a.cs == 1 && p.K >= 4 &&
+                       ((uintptr_t)p.a.p & 3) == 0 && p.a_bytes > 0 && p.a_bytes < kMaxRes;
+    const bool split_ok = planes != nullptr && (dma_ok || loose) && batch == 1 && p.b.kind == MGC_OP_STRIDED &&
+                          p.b.rs == 1 && (am != AM_CONV_VEC || p.a.cg % 8 == 0) && plane_data_bytes(p.N, p.K) < kMaxRes;
+    const int am_split = loose ? (int)AM_LOOSE : am;
 
     // The kernel family and K split: the library's choice from the shape, or the caller's
     // (g->kernel, g->split_k), checked against what that family accepts.
     int fam;
     SplitChoice sc{0, 0, 0};
-    if (g->kernel == MGC_GEMM_AUTO && split_ok && g->split_k <= 0)
+    if (g->kernel == MGC_GEMM_AUTO && split_ok && (g->split_k <= 0 || ln))
         sc = split_choice(p.M, p.N, p.K, g->workspace == nullptr ? 0 : g->workspace_floats, ln ? p.split : 0);
     if (sc.bm) {
-        fam = sc.bn == 64 ? MGC_GEMM_SPLIT_128X64 : MGC_GEMM_SPLIT_128X128;
+        fam = sc.bm == 32 ? (sc.bn == 64 ? MGC_GEMM_SPLIT_32X64 : MGC_GEMM_SPLIT_32X32)
+              : sc.bn == 64 ? MGC_GEMM_SPLIT_128X64 : MGC_GEMM_SPLIT_128X128;
         p.split = sc.split;
     } else if (g->kernel == MGC_GEMM_AUTO || ln) {
         if (stream_ok && g->split_k <= 0 &&
@@ -3375,15 +3407,15 @@ static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTai
         fam = g->kernel;
         const int split = g->split_k > 1 ? g->split_k : 1;
         const char *why = nullptr;
-        const bool split_fam = fam >= MGC_GEMM_SPLIT_128X128 && fam <= MGC_GEMM_SPLIT_128X64;
-        if (fam < MGC_GEMM_TILED || fam > MGC_GEMM_SPLIT_128X64)
+        const bool split_fam = fam >= MGC_GEMM_SPLIT_128X128 && fam <= MGC_GEMM_SPLIT_32X32;
+        if (fam < MGC_GEMM_TILED || fam > MGC_GEMM_SPLIT_32X32)
             why = "unknown kernel family";
         else if (split_fam && !split_ok)
             why = "the bf16-split kernels need planes of B (mgc_hip_gemm_planes), batch 1, k-contiguous operands below "
                   "2 GiB and convolution groups of a multiple of 8 channels";
         else if (split > 1 && (batch != 1 || g->workspace == nullptr || g->workspace_floats < (long)split * p.M * p.N))
             why = "a K split needs batch 1 and split_k * M * N floats of workspace";
-        else if (fam != MGC_GEMM_REGISTER && fam != MGC_GEMM_STREAM && !dma_ok)
+        else if (!split_fam && fam != MGC_GEMM_REGISTER && fam != MGC_GEMM_STREAM && !dma_ok)
             why = "the DMA kernels need k-contiguous operands (row-major A or NHWC image with 16-byte rows, "
                   "packed [N][K] B, K % 4 == 0) below 2 GiB";
         else if (fam == MGC_GEMM_QUARTER && (split > 1 || batch != 1 || !quarter_tiles_ok(am, p)))
@@ -3414,8 +3446,10 @@ static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTai
     p.kchunk = ((p.K + p.split - 1) / p.split + 31) / 32 * 32;
     if (p.kchunk == 0) p.kchunk = 32;
     const bool split_fam = fam >= MGC_GEMM_SPLIT_128X128;
-    const int bn_s = fam == MGC_GEMM_SPLIT_128X128 ? 128 : 64;
-    const int bm_t = split_fam ? 128 : fam == MGC_GEMM_WSPLIT16 ? 16 : fam == MGC_GEMM_WSPLIT ? 32 : fam == MGC_GEMM_NARROW ? 128 : 64;
+    if (fam == MGC_GEMM_SPLIT_32X64 && loose) fam = MGC_GEMM_SPLIT_32X32;  // the only 32-row form of a loose A
+    const int bm_s = fam <= MGC_GEMM_SPLIT_128X64 ? 128 : 32;
+    const int bn_s = fam == MGC_GEMM_SPLIT_128X128 ? 128 : fam == MGC_GEMM_SPLIT_32X32 ? 32 : 64;
+    const int bm_t = split_fam ? bm_s : fam == MGC_GEMM_WSPLIT16 ? 16 : fam == MGC_GEMM_WSPLIT ? 32 : fam == MGC_GEMM_NARROW ? 128 : 64;
     const int bn_t = split_fam ? bn_s : fam == MGC_GEMM_WSPLIT16 ? 16 : fam == MGC_GEMM_WSPLIT || fam == MGC_GEMM_NARROW ? 32 : 64;
     p.tiles_m = (p.M + bm_t - 1) / bm_t;
     p.tiles_n = (p.N + bn_t - 1) / bn_t;
@@ -3435,7 +3469,7 @@ static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTai
         return;
     }
     if (split_fam) {
-        MGC_LAUNCH(x, pick_split(am, bn_s), grid, dim3(256), 0, p, static_cast<const unsigned char *>(planes),
+        MGC_LAUNCH(x, pick_split(am_split, bm_s, bn_s), grid, dim3(bm_s == 32 ? 512 : 256), 0, p, static_cast<const unsigned char *>(planes),
                    plane_data_bytes(p.N, p.K), plane_kblocks(p.K));
     } else {
         MGC_LAUNCH(x, kern, grid, dim3(threads), 0, p);

@@ -7,9 +7,13 @@ namespace mgc {
 
 typedef void (*SplitKernel)(const GemmDev, const unsigned char *planes, long plane_bytes, int kblocks);
 
-// The kernel for 128 x bn tiles (bn 128 or 64) of an A operand of form am (AM_VEC, AM_CONV_VEC
-// or AM_CAT).
-SplitKernel pick_split(int am, int bn);
+// A row-major A that is only 4-byte aligned (its row stride or K no multiple of four), beside the
+// AM_* forms of gemm_device.h.
+enum { AM_LOOSE = 4 };
+
+// The kernel for bm x bn tiles (128 x 128, 128 x 64, 32 x 64 or 32 x 32) of an A operand of form am
+// (AM_VEC, AM_CONV_VEC, AM_CAT or AM_LOOSE).
+SplitKernel pick_split(int am, int bm, int bn);
 
 // Tile and K split of a GEMM on the bf16-split kernels; bm 0: the fp32 kernels are faster.
 struct SplitChoice {

@@ -61,7 +61,7 @@ __device__ __forceinline__ float dot_fp32(const GemmDev &p, const float *abase, 
     float sum = 0.0f;
     const mgc_hip_operand &img = AMODE == AM_CAT ? p.a2 : p.a;
     int n = 0, oh = 0, ow = 0;
-    if (AMODE != AM_VEC) {
+    if (AMODE == AM_CONV_VEC || AMODE == AM_CAT) {
         n = fdiv(row, p.div_ohw);
         const int rr = row - n * img.OH * img.OW;
         oh = fdiv(rr, p.div_ow);
@@ -71,8 +71,7 @@ __device__ __forceinline__ float dot_fp32(const GemmDev &p, const float *abase, 
     for (int k = kbeg; k < kend; ++k) {
         float a;
         if (AMODE == AM_CONV_VEC) {
-            const int t = fdiv(k, p.div_cg);
-            const int kh = fdiv(t, p.div_kw);
+            const int t = fdiv(k, p.div_cg), kh = fdiv(t, p.div_kw);
             const int ih = oh * p.a.SH - p.a.PT + kh * p.a.DH;
             const int iw = ow * p.a.SW - p.a.PL + (t - kh * p.a.KW) * p.a.DW;
             const bool ok = (unsigned)ih < (unsigned)p.a.H && (unsigned)iw < (unsigned)p.a.W;
@@ -129,6 +128,112 @@ __global__ void __launch_bounds__(256) tiny_columns_kernel(const float *b, long 
     if (lane == 0) flags[n] = most > 0.0f && most < 0x1p-95f;
 }
 
+// One lane's row of A: 8 consecutive k at a time through a buffer resource, masked elements zero.
+template <int AMODE>
+struct SplitRow {
+    static constexpr unsigned OOB = 0x80000000u;  // past every resource's end (extents are < 2^31 bytes)
+    unsigned aoff = OOB, aoff2 = OOB;  // byte offset of the row (AM_CONV_VEC: of its window's origin; AM_CAT: in a2)
+    int aih = -0x40000000, aiw = -0x40000000;  // fails the window bounds test
+
+    __device__ __forceinline__ SplitRow(const GemmDev &p, int m) {
+        if (m >= p.M) return;
+        if (AMODE == AM_CAT) {
+            const int n = fdiv(m, p.div_ohw), rr = m - n * p.a2.OH * p.a2.OW;
+            const int oh = fdiv(rr, p.div_ow), ow = rr - oh * p.a2.OW;
+            aoff2 = (unsigned)(((n * p.a2.H + oh * p.a2.SH) * p.a2.W + ow * p.a2.SW) * p.a2.C) * 4u;
+        }
+        if (AMODE == AM_CONV_VEC) {
+            const int n = fdiv(m, p.div_ohw), rr = m - n * p.a.OH * p.a.OW;
+            const int oh = fdiv(rr, p.div_ow), ow = rr - oh * p.a.OW;
+            aih = oh * p.a.SH - p.a.PT;
+            aiw = ow * p.a.SW - p.a.PL;
+            aoff = (unsigned)(((n * p.a.H + aih) * p.a.W + aiw) * p.a.C) * 4u;
+        } else {
+            aoff = (unsigned)m * (unsigned)p.a.rs * 4u;
+        }
+    }
+
+    // Four k of a row that is only 4-byte aligned: the load stays inside the row (the last four
+    // elements where k is nearer its end) and the elements are moved into place.
+    __device__ __forceinline__ f4 load_loose(__amdgpu_buffer_rsrc_t r, int k, int kend) const {
+        const int at = min(k, kend - 4), s = k - at;
+        const f4 v = buf_load4(r, s < 4 ? aoff + (unsigned)at * 4u : OOB);
+        const f4 t = {s & 1 ? v[1] : v[0], s & 1 ? v[2] : v[1], s & 1 ? v[3] : v[2], s & 1 ? 0.0f : v[3]};
+        return f4{s & 2 ? t[2] : t[0], s & 2 ? t[3] : t[1], s & 2 ? 0.0f : t[2], s & 2 ? 0.0f : t[3]};
+    }
+
+    // x, y: elements k .. k + 3 and k + 4 .. k + 7 (k a multiple of 8) of a stage that starts at `stage`.
+    __device__ __forceinline__ void load(const GemmDev &p, int stage, int k, int kend, f4 &x, f4 &y) const {
+        const bool k0 = k < kend, k1 = k + 4 < kend;
+        if constexpr (AMODE == AM_CAT) {
+            // k1 is a multiple of the 32-wide stage, so a whole stage reads one source
+            const bool second = stage >= p.k1;
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+                (void *)(second ? p.a2.p : p.a.p), (short)0, (int)(second ? p.a2_bytes : p.a_bytes), 0x00020000);
+            const unsigned o = second ? aoff2 + (unsigned)(k - p.k1) * 4u : aoff + (unsigned)k * 4u;
+            x = buf_load4(r, k0 ? o : OOB);
+            y = buf_load4(r, k1 ? o + 16u : OOB);
+        } else {
+            const __amdgpu_buffer_rsrc_t r =
+                __builtin_amdgcn_make_buffer_rsrc((void *)p.a.p, (short)0, (int)p.a_bytes, 0x00020000);
+            if constexpr (AMODE == AM_VEC) {
+                const unsigned o = aoff + (unsigned)k * 4u;
+                x = buf_load4(r, k0 ? o : OOB);
+                y = buf_load4(r, k1 ? o + 16u : OOB);
+            } else if constexpr (AMODE == AM_LOOSE) {
+                x = load_loose(r, k, kend);
+                y = load_loose(r, k + 4, kend);
+            } else {  // cg % 8 == 0: the 8 k share a tap
+                const int t = fdiv(k, p.div_cg), kh = fdiv(t, p.div_kw);
+                const int dh = kh * p.a.DH, dw = (t - kh * p.a.KW) * p.a.DW;
+                const bool ok = k0 && (unsigned)(aih + dh) < (unsigned)p.a.H && (unsigned)(aiw + dw) < (unsigned)p.a.W;
+                const unsigned o = ok ? aoff + (unsigned)((dh * p.a.W + dw) * p.a.C + (k - t * p.a.cg)) * 4u : OOB;
+                x = buf_load4(r, o);
+                y = buf_load4(r, o + 16u);
+            }
+        }
+    }
+};
+
+// Eight consecutive k of a row as the three MFMA operands; `seen` collects the magnitude bits of
+// the leading parts.
+__device__ __forceinline__ void split_row(const f4 &x, const f4 &y, bf8 (&a)[3], unsigned &seen) {
+    uint4_t h, m, l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const f4 &v = e < 2 ? x : y;
+        unsigned u0, u1, u2;
+        split3(v[2 * (e & 1)], v[2 * (e & 1) + 1], u0, u1, u2);
+        h[e] = u0;
+        m[e] = u1;
+        l[e] = u2;
+    }
+    seen |= (h[0] | h[1]) | (h[2] | h[3]);
+    a[0] = __builtin_bit_cast(bf8, h);
+    a[1] = __builtin_bit_cast(bf8, m);
+    a[2] = __builtin_bit_cast(bf8, l);
+}
+
+// Whether the elements that `seen` was collected from are all below 2^-95 and not all zero (bf16
+// exponent bits of the OR below 32): their low parts are out of bf16's range.
+__device__ __forceinline__ bool tiny_row(unsigned seen) { return ((seen | (seen >> 16)) & 0x7fffu) - 1u < 0x0fffu; }
+
+// Replace the sums of one 16-byte chunk (row, columns col ..) that the split cannot have right.
+template <int AMODE>
+__device__ __forceinline__ void fix_sums(const GemmDev &p, f4 &v, unsigned mark, int row, int col, int ncol, int kbeg,
+                                         int kend) {
+    const float z = (v[0] * 0.0f + v[1] * 0.0f) + (v[2] * 0.0f + v[3] * 0.0f);  // NaN if a sum is not finite
+    if (z == z && !mark) return;
+#pragma unroll 1
+    for (int e = 0; e < ncol; ++e) {
+        const float s = dot_fp32<AMODE>(p, p.a.p, p.b.p, row, col + e, kbeg, kend);
+        v[0] = e == 0 ? s : v[0];
+        v[1] = e == 1 ? s : v[1];
+        v[2] = e == 2 ? s : v[2];
+        v[3] = e == 3 ? s : v[3];
+    }
+}
+
 // A workgroup of WAVES waves owns a tile of 32 WAVES rows x 32 RN columns; each wave owns 32 rows and
 // all the columns. K advances 32 per stage (two MFMA depths of 16).
 //
@@ -175,82 +280,19 @@ __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
     const int kbeg = ks * p.kchunk;
     const int kend = min(p.K, kbeg + p.kchunk);
     const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
-    constexpr unsigned OOB = 0x80000000u;  // past every resource's end (extents are < 2^31 bytes)
+    constexpr unsigned OOB = SplitRow<AMODE>::OOB;
 
-    // ---- A: this lane's row and its 8 k of each 16 -----------------------------------------
     const int li = lane & 31;
     const int lh = lane >> 5;
-    const __amdgpu_buffer_rsrc_t ra =
-        __builtin_amdgcn_make_buffer_rsrc((void *)p.a.p, (short)0, (int)p.a_bytes, 0x00020000);
-    unsigned aoff = OOB, aoff2 = OOB;
-    int aih = -0x40000000, aiw = -0x40000000;  // fails the window bounds test
-    {
-        const int m = m0 + 32 * wave + li;
-        if (m < p.M) {
-            if (AMODE == AM_CAT) {
-                const int n = fdiv(m, p.div_ohw), rr = m - n * p.a2.OH * p.a2.OW;
-                const int oh = fdiv(rr, p.div_ow), ow = rr - oh * p.a2.OW;
-                aoff2 = (unsigned)(((n * p.a2.H + oh * p.a2.SH) * p.a2.W + ow * p.a2.SW) * p.a2.C) * 4u;
-            }
-            if (AMODE == AM_CONV_VEC) {
-                const int n = fdiv(m, p.div_ohw), rr = m - n * p.a.OH * p.a.OW;
-                const int oh = fdiv(rr, p.div_ow), ow = rr - oh * p.a.OW;
-                aih = oh * p.a.SH - p.a.PT;
-                aiw = ow * p.a.SW - p.a.PL;
-                aoff = (unsigned)(((n * p.a.H + aih) * p.a.W + aiw) * p.a.C) * 4u;
-            } else {
-                aoff = (unsigned)m * (unsigned)p.a.rs * 4u;
-            }
-        }
-    }
-    f4 va[2][4];        // [set][16-k block, half of the lane's 8 k]
-    int ka = kbeg;      // the stage the next A loads fetch
+    const SplitRow<AMODE> arow(p, m0 + 32 * wave + li);
+    f4 va[2][4];    // [set][16-k block, half of the lane's 8 k]
+    int ka = kbeg;  // the stage the next A loads fetch
     auto load_a = [&](f4 (&v)[4]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const int k = ka + 16 * s + 8 * lh;
-            const bool k0 = k < kend, k1 = k + 4 < kend;
-            if constexpr (AMODE == AM_VEC) {
-                const unsigned o = aoff + (unsigned)k * 4u;
-                v[2 * s] = buf_load4(ra, k0 ? o : OOB);
-                v[2 * s + 1] = buf_load4(ra, k1 ? o + 16u : OOB);
-            } else if constexpr (AMODE == AM_CAT) {
-                // k1 is a multiple of the 32-wide stage, so a whole stage reads one source
-                const bool second = ka >= p.k1;
-                const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-                    (void *)(second ? p.a2.p : p.a.p), (short)0, (int)(second ? p.a2_bytes : p.a_bytes), 0x00020000);
-                const unsigned o = second ? aoff2 + (unsigned)(k - p.k1) * 4u : aoff + (unsigned)k * 4u;
-                v[2 * s] = buf_load4(r, k0 ? o : OOB);
-                v[2 * s + 1] = buf_load4(r, k1 ? o + 16u : OOB);
-            } else {  // cg % 8 == 0: the 8 k share a tap
-                const int t = fdiv(k, p.div_cg), kh = fdiv(t, p.div_kw);
-                const int dh = kh * p.a.DH, dw = (t - kh * p.a.KW) * p.a.DW;
-                const bool ok = k0 && (unsigned)(aih + dh) < (unsigned)p.a.H && (unsigned)(aiw + dw) < (unsigned)p.a.W;
-                const unsigned o =
-                    ok ? aoff + (unsigned)((dh * p.a.W + dw) * p.a.C + (k - t * p.a.cg)) * 4u : OOB;
-                v[2 * s] = buf_load4(ra, o);
-                v[2 * s + 1] = buf_load4(ra, o + 16u);
-            }
-        }
+        for (int s = 0; s < 2; ++s) arow.load(p, ka, ka + 16 * s + 8 * lh, kend, v[2 * s], v[2 * s + 1]);
         ka += BK;
     };
-    unsigned seen = 0;  // magnitude bits of the row's leading parts (see below)
-    auto split_a = [&](const f4 &x, const f4 &y, bf8 (&a)[3]) __attribute__((always_inline)) {
-        uint4_t h, m, l;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const f4 &v = e < 2 ? x : y;
-            unsigned u0, u1, u2;
-            split3(v[2 * (e & 1)], v[2 * (e & 1) + 1], u0, u1, u2);
-            h[e] = u0;
-            m[e] = u1;
-            l[e] = u2;
-        }
-        seen |= (h[0] | h[1]) | (h[2] | h[3]);
-        a[0] = __builtin_bit_cast(bf8, h);
-        a[1] = __builtin_bit_cast(bf8, m);
-        a[2] = __builtin_bit_cast(bf8, l);
-    };
+    unsigned seen = 0;
 
     // ---- B: 1 KB copy c of a stage is plane c % 3 of 16-k block c / 3 % 2 of column block c / 6 ----
     const __amdgpu_buffer_rsrc_t rb =
@@ -282,7 +324,7 @@ __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
     auto step = [&](const bf8 (&a)[3], const unsigned char *bs, const f4 &x, const f4 &y, bf8 (&next)[3])
                     __attribute__((always_inline)) {
         constexpr int G = RN < 2 ? RN : 2;  // column blocks at a time: independent chains, few registers
-        split_a(x, y, next);
+        split_row(x, y, next, seen);
 #pragma unroll
         for (int j0 = 0; j0 < RN; j0 += G) {
             bf8 b[G][3];
@@ -326,7 +368,7 @@ __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
     copy_b(1);
     load_a(va[1]);
     asm volatile("" ::: "memory");
-    split_a(va[0][0], va[0][1], a0);
+    split_row(va[0][0], va[0][1], a0, seen);
     for (int kt = nk >> 1; kt > 0; --kt) {
         stage(va[0], va[1]);
         stage(va[1], va[0]);
@@ -335,9 +377,7 @@ __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
     wait_vmcnt<0>();  // masked copies past the end may still be writing the ring
     __syncthreads();
 
-    // A row whose elements (as this lane saw them: a half of its k) are all below 2^-95 and not
-    // all zero: bf16 exponent bits of the OR below 32.
-    if (((seen | (seen >> 16)) & 0x7fffu) - 1u < 0x0fffu) flags[32 * wave + li] = 1;
+    if (tiny_row(seen)) flags[32 * wave + li] = 1;  // as this lane saw the row: a half of its k
     float *const Cs = reinterpret_cast<float *>(smem);
 #pragma unroll
     for (int j = 0; j < RN; ++j) {
@@ -349,29 +389,205 @@ __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
     __syncthreads();
     const unsigned char *const cflags = planes + plane_bytes;
     const auto fix = [&](f4 &v, int rl, int cl, int ncol) __attribute__((always_inline)) {
-        const float z = (v[0] * 0.0f + v[1] * 0.0f) + (v[2] * 0.0f + v[3] * 0.0f);  // NaN if a sum is not finite
         const unsigned mark = flags[rl] | *reinterpret_cast<const unsigned *>(cflags + n0 + cl);
-        if (z != z || mark) {
-#pragma unroll 1
-            for (int e = 0; e < ncol; ++e) {
-                const float s = dot_fp32<AMODE>(p, p.a.p, p.b.p, m0 + rl, n0 + cl + e, kbeg, kend);
-                v[0] = e == 0 ? s : v[0];
-                v[1] = e == 1 ? s : v[1];
-                v[2] = e == 2 ? s : v[2];
-                v[3] = e == 3 ? s : v[3];
-            }
-        }
+        fix_sums<AMODE>(p, v, mark, m0 + rl, n0 + cl, ncol, kbeg, kend);
     };
     gemm_lds_to_global<BM, BN, decltype(fix), 64 * WAVES>(p, Cs, m0, n0, ks, 0, 0, fix);
 }
 
-template <int RN, int WAVES>
-static SplitKernel pick(int am) {
-    return am == AM_VEC   ? &gemm_split_kernel<RN, WAVES, 3, AM_VEC>
-           : am == AM_CAT ? &gemm_split_kernel<RN, WAVES, 3, AM_CAT>
-                          : &gemm_split_kernel<RN, WAVES, 3, AM_CONV_VEC>;
+// The same products for GEMMs whose 128-row tiles are too few for the CUs: a tile of 32 rows x 32 RN
+// columns per workgroup, whose K stages are dealt to its WAVES waves (wave w takes stages w,
+// w + WAVES, ...). Every wave loads its own A rows and B planes straight into registers, two stages
+// ahead, so the main loop has neither LDS nor barriers; a stage's B planes are linear 1 KB loads.
+// The partial tiles are summed through LDS in wave order, each thread finishing the 16-byte chunks
+// whose bias and residual it requested at the start.
+template <int RN, int WAVES, int AMODE>
+__global__ void __launch_bounds__(64 * WAVES)
+    gemm_split_small_kernel(const GemmDev p, const unsigned char *planes, long plane_bytes, int kblocks) {
+    constexpr int BK = 32, T = 32;
+    constexpr int BN = 32 * RN;
+    constexpr int LDC = BN + 8;
+    constexpr int CHUNKS = T * BN / 4;                      // 16-byte chunks of the tile
+    constexpr int PER = (CHUNKS + 64 * WAVES - 1) / (64 * WAVES);  // per thread
+    constexpr int FLAGS = WAVES * T * LDC * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[FLAGS + T];
+    unsigned char *const flags = smem + FLAGS;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb = gridDim.x;
+    const int full = nb & ~7;
+    int lin = blockIdx.x;
+    if (lin < full) {
+        const int per = full >> 3;
+        lin = (lin & 7) * per + (lin >> 3);
+    }
+    // rows fastest: the workgroups that share B planes (the larger operand here) are neighbours
+    const int tn = lin / p.tiles_m;
+    const int tm = lin - tn * p.tiles_m;
+    const int m0 = tm * T, n0 = tn * BN;
+    const int ks = blockIdx.z;
+    const int kbeg = ks * p.kchunk;
+    const int kend = min(p.K, kbeg + p.kchunk);
+    const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
+    const int nkw = nk > wave ? (nk - 1 - wave) / WAVES + 1 : 0;  // this wave's stages
+
+    const int li = lane & 31;
+    const int lh = lane >> 5;
+    const SplitRow<AMODE> arow(p, m0 + li);
+    const __amdgpu_buffer_rsrc_t rb =
+        __builtin_amdgcn_make_buffer_rsrc((void *)planes, (short)0, (int)plane_bytes, 0x00020000);
+    unsigned boff[RN];  // column blocks past N lie past the resource's end, whatever stage is added
+#pragma unroll
+    for (int j = 0; j < RN; ++j) {
+        const int block = n0 / 32 + j;
+        boff[j] = block * 32 < p.N ? ((unsigned)block * (unsigned)kblocks + (unsigned)((kbeg >> 4) + 2 * wave)) * 3072u +
+                                         (unsigned)lane * 16u
+                                   : SplitRow<AMODE>::OOB;
+    }
+    int ka = kbeg + wave * BK;
+    f4 va[2][4], vb[2][RN][6];
+    auto load = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            arow.load(p, ka, ka + 16 * s + 8 * lh, kend, va[set][2 * s], va[set][2 * s + 1]);
+        const bool live = ka < kend;  // stages past the end read nothing
+#pragma unroll
+        for (int j = 0; j < RN; ++j) {
+            const unsigned o = live ? boff[j] : SplitRow<AMODE>::OOB;
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+                vb[set][j][q] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)o, q * 1024, 0));
+            boff[j] += (unsigned)WAVES * 6144u;
+        }
+        ka += WAVES * BK;
+    };
+    load(0);
+    load(1);
+
+    // epilogue operands: thread t owns chunks t, t + 64 WAVES, ...
+    const bool split_out = p.split > 1;
+    const bool vec = split_out ? p.N % 4 == 0 : p.vec_out != 0;
+    const f4 zero4 = {0.f, 0.f, 0.f, 0.f};
+    f4 ebias[PER], eres[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int c = tid + u * 64 * WAVES;
+        const int row = m0 + c / (BN / 4), col = n0 + c % (BN / 4) * 4;
+        ebias[u] = eres[u] = zero4;
+        if (c < CHUNKS && row < p.M && col + 4 <= p.N && vec && !split_out) {
+            if (p.bias && p.bias_mode == 1) ebias[u] = ldg4(p.bias + col);
+            if (p.res) eres[u] = ldg4(p.res + (long)row * p.ldr + col);
+        }
+    }
+    if (tid < T) flags[tid] = 0;
+
+    floatx16 acc[RN], cor[RN];
+#pragma unroll
+    for (int j = 0; j < RN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[j][r] = cor[j][r] = 0.0f;
+    unsigned seen = 0;
+    auto stage = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            bf8 a[3];
+            split_row(va[set][2 * s], va[set][2 * s + 1], a, seen);
+#define MGC_MFMA(C, QA, QB)                                                                                        \
+    _Pragma("unroll") for (int j = 0; j < RN; ++j) C[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(                 \
+        a[QA], __builtin_bit_cast(bf8, vb[set][j][3 * s + QB]), C[j], 0, 0, 0);
+            MGC_MFMA(acc, 0, 0)
+            MGC_MFMA(cor, 2, 0)
+            MGC_MFMA(cor, 1, 0)
+            MGC_MFMA(cor, 1, 1)
+            MGC_MFMA(cor, 0, 1)
+            MGC_MFMA(cor, 0, 2)
+#undef MGC_MFMA
+        }
+        load(set);
+    };
+    for (int kt = nkw >> 1; kt > 0; --kt) {
+        stage(0);
+        stage(1);
+    }
+    if (nkw & 1) stage(0);
+
+    float *const slots = reinterpret_cast<float *>(smem);
+#pragma unroll
+    for (int j = 0; j < RN; ++j) {
+        acc[j] += cor[j];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            slots[wave * (T * LDC) + ((r >> 2) * 8 + lh * 4 + (r & 3)) * LDC + j * 32 + li] = acc[j][r];
+    }
+    __syncthreads();  // the flags are cleared
+    if (tiny_row(seen)) flags[li] = 1;
+    __syncthreads();
+    const unsigned char *const cflags = planes + plane_bytes;
+    const int M = p.M, N = p.N, act = p.act, bias_mode = p.bias ? p.bias_mode : 0;
+    const float alpha = p.alpha, beta = p.beta, lo = p.lo, hi = p.hi;
+    const float *const bias = p.bias, *const res = p.res;
+    const long ldr = p.ldr;
+    float *const cbase = split_out ? p.ws + (long)ks * M * N : p.c;
+    const long ldc = split_out ? (long)N : p.ldc;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int c = tid + u * 64 * WAVES;
+        const int rl = c / (BN / 4), cl = c % (BN / 4) * 4;
+        const int row = m0 + rl, col = n0 + cl;
+        if (c >= CHUNKS || row >= M || col >= N) continue;
+        const int ncol = min(4, N - col);
+        const bool full4 = vec && ncol == 4;
+        const int o = rl * LDC + cl;
+        f4 v = *reinterpret_cast<const f4 *>(&slots[o]);
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) v += *reinterpret_cast<const f4 *>(&slots[w * (T * LDC) + o]);
+        fix_sums<AMODE>(p, v, flags[rl] | *reinterpret_cast<const unsigned *>(cflags + col), row, col, ncol, kbeg, kend);
+        float *const dst = cbase + (long)row * ldc + col;
+        if (!split_out) {
+            f4 b = ebias[u], r = eres[u];
+            if (!full4) {  // scalar bias and residual reads
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (e < ncol && bias_mode == 1) b[e] = ldg(bias + col + e);
+                    if (e < ncol && res) r[e] = ldg(res + (long)row * ldr + col + e);
+                }
+            }
+            v = v * alpha + b;
+            if (bias_mode == 2) v += ldg(bias + row);
+            if (res) v += beta * r;
+            v = act4(v, act, lo, hi);
+        }
+        if (full4) {
+            *reinterpret_cast<f4 *>(dst) = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (e < ncol) dst[e] = v[e];
+        }
+    }
 }
 
-SplitKernel pick_split(int am, int bn) { return bn == 128 ? pick<4, 4>(am) : pick<2, 4>(am); }
+template <int RN>
+static SplitKernel pick(int am) {
+    return am == AM_VEC     ? &gemm_split_kernel<RN, 4, 3, AM_VEC>
+           : am == AM_CAT   ? &gemm_split_kernel<RN, 4, 3, AM_CAT>
+           : am == AM_LOOSE ? &gemm_split_kernel<RN, 4, 3, AM_LOOSE>
+                            : &gemm_split_kernel<RN, 4, 3, AM_CONV_VEC>;
+}
+
+template <int RN, int WAVES>
+static SplitKernel pick_small(int am) {
+    return am == AM_VEC   ? &gemm_split_small_kernel<RN, WAVES, AM_VEC>
+           : am == AM_CAT ? &gemm_split_small_kernel<RN, WAVES, AM_CAT>
+                          : &gemm_split_small_kernel<RN, WAVES, AM_CONV_VEC>;
+}
+
+SplitKernel pick_split(int am, int bm, int bn) {
+    if (bm == 32 && am == AM_LOOSE) return &gemm_split_small_kernel<1, 8, AM_LOOSE>;  // bn 32 only: registers
+    if (bm == 32) return bn == 64 ? pick_small<2, 8>(am) : pick_small<1, 8>(am);
+    return bn == 128 ? pick<4>(am) : pick<2>(am);
+}
 
 }  // namespace mgc

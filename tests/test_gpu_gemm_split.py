@@ -1,8 +1,8 @@
 """fp32 GEMMs on the bf16 matrix cores (mgc_hip_gemm_planes) against float64.
 
-Both tile shapes are pinned through mgc_hip_gemm_args.kernel at the edges of their tiles (128 rows,
-64 or 128 columns, 32 k per stage, 16 k per MFMA), for row-major A, NHWC convolutions and a
-concatenated K, with a K split and a rotating epilogue. The tolerance is the standard bound of a
+Every tile shape is pinned through mgc_hip_gemm_args.kernel at the edges of its tiles (128 or 32
+rows, 32 to 128 columns, 32 k per stage, 16 k per MFMA, eight waves sharing K), for row-major A, also
+of rows that are only 4-byte aligned (K no multiple of four), NHWC convolutions and a concatenated K, with a K split and a rotating epilogue. The tolerance is the standard bound of a
 summation: with S = sum |a||b| of an element, at most 6 K / 16 + 8 roundings of 2^-24 S for the MFMA
 accumulations and the epilogue, and 2^-23 S for the products the split drops.
 
@@ -23,7 +23,7 @@ from oracle import interpreter as oracle
 
 pytestmark = pytest.mark.gpu
 
-FAMILIES = {"128x128": 8, "128x64": 9}
+FAMILIES = {"128x128": 8, "128x64": 9, "32x64": 10, "32x32": 11}
 
 
 class Runner:
@@ -88,16 +88,18 @@ def _bound(a64: np.ndarray, b64: np.ndarray, k: int) -> np.ndarray:
     return (6 * k / 16 + 10) * 2.0**-24 * s
 
 
-def _check(got, a64, b64, extra=0.0, bias=None, bias_mode=0, res=None, alpha=1.0, beta=1.0, act="none"):
+def _check(got, a64, b64, bias=None, bias_mode=0, res=None, alpha=1.0, beta=1.0, act="none"):
     y = alpha * (a64 @ b64.T)
     scale = abs(alpha) * _bound(a64, b64, a64.shape[1])
-    if bias_mode == 1:
-        y = y + bias[None, :].astype(np.float64)
-    if bias_mode == 2:
-        y = y + bias[:, None].astype(np.float64)
+    # the epilogue's own roundings (alpha, bias, beta, residual: four of 2^-24) are of partial sums,
+    # whose size the terms' sizes bound where they cancel in y
+    terms = np.abs(y)
+    if bias_mode:
+        b = bias[None, :] if bias_mode == 1 else bias[:, None]
+        y, terms = y + b.astype(np.float64), terms + np.abs(b)
     if res is not None:
-        y = y + beta * res.astype(np.float64)
-    scale = scale + 2.0**-22 * np.abs(y) + 1e-30 + extra  # the epilogue's own roundings
+        y, terms = y + beta * res.astype(np.float64), terms + np.abs(beta * res)
+    scale = scale + 2.0**-22 * terms + 1e-30
     if act != "none":
         y = oracle.activation(y, {"activation": act, "clip_min": -0.5, "clip_max": 0.75})
         scale = 1.2 * scale + 5e-7  # slope at most 1.13 (GELU), the activations' own approximation
@@ -105,7 +107,7 @@ def _check(got, a64, b64, extra=0.0, bias=None, bias_mode=0, res=None, alpha=1.0
 
 
 @pytest.mark.parametrize("family", FAMILIES)
-@pytest.mark.parametrize("k", [4, 16, 28, 32, 36, 64, 68, 100, 260, 1028])
+@pytest.mark.parametrize("k", [4, 16, 28, 32, 36, 64, 68, 100, 260, 1028, 5, 7, 30, 33, 65, 99, 259])
 def test_shapes(runner, family, k):
     """Rows and columns at the tiles' edges, K at the stages', every epilogue and K splits."""
     rng = np.random.default_rng(k)
@@ -220,8 +222,9 @@ def test_refusals(runner):
     g.c, g.ldc, g.kernel = runner.hip.empty(4 * 128 * 64), 64, 9
     runner.lib.mgc_hip_gemm(runner.x, ctypes.byref(g))
     assert runner.lib.mgc_hip_exec_status(runner.x) == MGC_ERR_ARGS
-    g.a.p = g.a.p + 4  # not 16-byte aligned: refused when pinned, fp32 kernels otherwise
-    g.M = 127
+    g.M, g.a.p = 127, g.a.p + 4  # only 4-byte aligned: read element-aligned
+    assert runner.run(g, planes) == MGC_OK
+    g.a.cs, g.a.rs, g.M = 4, 1, 8  # columns apart: refused when pinned, fp32 kernels otherwise
     assert runner.run(g, planes) == MGC_ERR_ARGS
     g.kernel = 0
     assert runner.run(g, planes) == MGC_OK
