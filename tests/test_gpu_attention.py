@@ -204,6 +204,18 @@ def test_causal_and_biased_many_heads(hip_cache):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("fill", [-1e4, -np.inf, -3.0], ids=["finite", "inf", "near"])
+@pytest.mark.parametrize("B, H, S", [(1, 3, 129), (1, 7, 577), (5, 9, 450), (4, 13, 512), (37, 7, 130)])
+def test_causal_key_groups(B, H, S, fill, hip_cache):
+    """Causal masks on both sides of the rule for two key groups (9, 70, 360 and 416 workgroups
+    with them, 777 without), odd and even key-block
+    counts, heads that are no multiple of the 8 XCDs. A fill of -3 is within reach of the scores, so
+    no block past the diagonal may be skipped."""
+    g, feeds = attention_graph(B, H, S, S, 64, True, mask="causal", fill=fill)
+    _check(g, feeds, hip_cache)
+
+
+@pytest.mark.gpu
 def test_attention_outside_limits_stays_unfused(hip_cache):
     g, feeds = attention_graph(1, 2, 16, 40, 80, False)  # D > 64
     _check(g, feeds, hip_cache, fused=False)
