@@ -3361,7 +3361,8 @@ static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTai
                        ((uintptr_t)p.a.p & 3) == 0 && p.a_bytes > 0 && p.a_bytes < kMaxRes;
     const bool split_ok = planes != nullptr && (dma_ok || loose) && batch == 1 && p.b.kind == MGC_OP_STRIDED &&
                           p.b.rs == 1 && (am != AM_CONV_VEC || p.a.cg % 8 == 0) && plane_data_bytes(p.N, p.K) < kMaxRes;
-    const int am_split = loose ? (int)AM_LOOSE : am;
+    const bool tap = am == AM_CONV_VEC && p.a.cg % 32 == 0 && p.K == p.a.KH * p.a.KW * p.a.cg;
+    const int am_split = loose ? (int)AM_LOOSE : tap ? (int)AM_TAP : am;
 
     // The kernel family and K split: the library's choice from the shape, or the caller's
     // (g->kernel, g->split_k), checked against what that family accepts.

@@ -61,7 +61,7 @@ __device__ __forceinline__ float dot_fp32(const GemmDev &p, const float *abase, 
     float sum = 0.0f;
     const mgc_hip_operand &img = AMODE == AM_CAT ? p.a2 : p.a;
     int n = 0, oh = 0, ow = 0;
-    if (AMODE == AM_CONV_VEC || AMODE == AM_CAT) {
+    if (is_conv(AMODE) || AMODE == AM_CAT) {
         n = fdiv(row, p.div_ohw);
         const int rr = row - n * img.OH * img.OW;
         oh = fdiv(rr, p.div_ow);
@@ -70,7 +70,7 @@ __device__ __forceinline__ float dot_fp32(const GemmDev &p, const float *abase, 
 #pragma unroll 1
     for (int k = kbeg; k < kend; ++k) {
         float a;
-        if (AMODE == AM_CONV_VEC) {
+        if (is_conv(AMODE)) {
             const int t = fdiv(k, p.div_cg), kh = fdiv(t, p.div_kw);
             const int ih = oh * p.a.SH - p.a.PT + kh * p.a.DH;
             const int iw = ow * p.a.SW - p.a.PL + (t - kh * p.a.KW) * p.a.DW;
@@ -132,7 +132,7 @@ __global__ void __launch_bounds__(256) tiny_columns_kernel(const float *b, long 
 template <int AMODE>
 struct SplitRow {
     static constexpr unsigned OOB = 0x80000000u;  // past every resource's end (extents are < 2^31 bytes)
-    unsigned aoff = OOB, aoff2 = OOB;  // byte offset of the row (AM_CONV_VEC: of its window's origin; AM_CAT: in a2)
+    unsigned aoff = OOB, aoff2 = OOB;  // byte offset of the row (convolutions: of its window's origin; AM_CAT: in a2)
     int aih = -0x40000000, aiw = -0x40000000;  // fails the window bounds test
 
     __device__ __forceinline__ SplitRow(const GemmDev &p, int m) {
@@ -142,7 +142,7 @@ struct SplitRow {
             const int oh = fdiv(rr, p.div_ow), ow = rr - oh * p.a2.OW;
             aoff2 = (unsigned)(((n * p.a2.H + oh * p.a2.SH) * p.a2.W + ow * p.a2.SW) * p.a2.C) * 4u;
         }
-        if (AMODE == AM_CONV_VEC) {
+        if (is_conv(AMODE)) {
             const int n = fdiv(m, p.div_ohw), rr = m - n * p.a.OH * p.a.OW;
             const int oh = fdiv(rr, p.div_ow), ow = rr - oh * p.a.OW;
             aih = oh * p.a.SH - p.a.PT;
@@ -183,6 +183,18 @@ struct SplitRow {
             } else if constexpr (AMODE == AM_LOOSE) {
                 x = load_loose(r, k, kend);
                 y = load_loose(r, k + 4, kend);
+            } else if constexpr (AMODE == AM_TAP) {
+                // The stage's 32 k share a tap: its coordinates are scalar arithmetic, once a stage
+                // (211 vector instructions in two stages of 128 columns instead of 286, 24 of them
+                // multiplies at a quarter of the rate). ResNet-50 b32 2254 -> 2226 us.
+                const int t = fdiv(stage, p.div_cg), kh = fdiv(t, p.div_kw);
+                const int dh = kh * p.a.DH, dw = (t - kh * p.a.KW) * p.a.DW;
+                const bool ok =
+                    stage < kend && (unsigned)(aih + dh) < (unsigned)p.a.H && (unsigned)(aiw + dw) < (unsigned)p.a.W;
+                const int tap = (dh * p.a.W + dw) * p.a.C + (stage - t * p.a.cg);
+                const unsigned o = ok ? aoff + (unsigned)(tap + (k - stage)) * 4u : OOB;
+                x = buf_load4(r, o);
+                y = buf_load4(r, o + 16u);
             } else {  // cg % 8 == 0: the 8 k share a tap
                 const int t = fdiv(k, p.div_cg), kh = fdiv(t, p.div_kw);
                 const int dh = kh * p.a.DH, dw = (t - kh * p.a.KW) * p.a.DW;
@@ -574,6 +586,7 @@ static SplitKernel pick(int am) {
     return am == AM_VEC     ? &gemm_split_kernel<RN, 4, 3, AM_VEC>
            : am == AM_CAT   ? &gemm_split_kernel<RN, 4, 3, AM_CAT>
            : am == AM_LOOSE ? &gemm_split_kernel<RN, 4, 3, AM_LOOSE>
+           : am == AM_TAP   ? &gemm_split_kernel<RN, 4, 3, AM_TAP>
                             : &gemm_split_kernel<RN, 4, 3, AM_CONV_VEC>;
 }
 
@@ -581,6 +594,7 @@ template <int RN, int WAVES>
 static SplitKernel pick_small(int am) {
     return am == AM_VEC   ? &gemm_split_small_kernel<RN, WAVES, AM_VEC>
            : am == AM_CAT ? &gemm_split_small_kernel<RN, WAVES, AM_CAT>
+           : am == AM_TAP ? &gemm_split_small_kernel<RN, WAVES, AM_TAP>
                           : &gemm_split_small_kernel<RN, WAVES, AM_CONV_VEC>;
 }
 

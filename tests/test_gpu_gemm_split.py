@@ -134,6 +134,18 @@ def _im2col(x: np.ndarray, kh: int, stride: int, pad: int) -> np.ndarray:
 @pytest.mark.parametrize("family", FAMILIES)
 @pytest.mark.parametrize("c,kh,stride,pad,hw", [(8, 3, 1, 1, 9), (8, 3, 2, 0, 15), (24, 3, 1, 1, 7), (64, 3, 1, 1, 12), (64, 1, 2, 0, 14), (40, 5, 2, 2, 11)])
 def test_convolutions(runner, family, c, kh, stride, pad, hw):
+    _convolution(runner, family, c, kh, stride, pad, hw)
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+@pytest.mark.parametrize("c,kh,stride,pad,hw,split", [(32, 3, 1, 1, 9, 1), (32, 3, 2, 0, 11, 4), (96, 3, 2, 1, 9, 3), (64, 3, 1, 2, 6, 5), (160, 2, 1, 1, 5, 2)])
+def test_convolutions_one_tap_per_stage(runner, family, c, kh, stride, pad, hw, split):
+    """Channels in multiples of 32: a K stage reads one window tap; K splits start inside a tap's
+    channels (32 of 64 or 96) and at taps, the last part shorter or empty."""
+    _convolution(runner, family, c, kh, stride, pad, hw, split)
+
+
+def _convolution(runner, family, c, kh, stride, pad, hw, split=1):
     rng = np.random.default_rng(c + kh)
     x = rng.standard_normal((3, hw, hw, c)).astype(np.float32)
     cols = _im2col(x, kh, stride, pad)
@@ -152,7 +164,7 @@ def test_convolutions(runner, family, c, kh, stride, pad, hw):
         g.a.PT = g.a.PL = pad
         g.a.OH = g.a.OW = o
 
-    got = runner.gemm(family, x, b, fill=fill, m=m, act="relu")
+    got = runner.gemm(family, x, b, fill=fill, m=m, split=split, act="relu")
     _check(got, cols.astype(np.float64), b.astype(np.float64), act="relu")
 
 
