@@ -190,7 +190,7 @@ struct SplitRow {
                 const int t = fdiv(stage, p.div_cg), kh = fdiv(t, p.div_kw);
                 const int dh = kh * p.a.DH, dw = (t - kh * p.a.KW) * p.a.DW;
                 const bool ok =
-                    stage < kend && (unsigned)(aih + dh) < (unsigned)p.a.H && (unsigned)(aiw + dw) < (unsigned)p.a.W;
+                    (stage < kend) & ((unsigned)(aih + dh) < (unsigned)p.a.H) & ((unsigned)(aiw + dw) < (unsigned)p.a.W);
                 const int tap = (dh * p.a.W + dw) * p.a.C + (stage - t * p.a.cg);
                 const unsigned o = ok ? aoff + (unsigned)(tap + (k - stage)) * 4u : OOB;
                 x = buf_load4(r, o);
@@ -331,44 +331,97 @@ __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[j][r] = cor[j][r] = 0.0f;
 
-    // One 16-k step: multiply fragments a by the step's B while the next step's A (x, y) is split
-    // into `next`.
-    auto step = [&](const bf8 (&a)[3], const unsigned char *bs, const f4 &x, const f4 &y, bf8 (&next)[3])
-                    __attribute__((always_inline)) {
-        constexpr int G = RN < 2 ? RN : 2;  // column blocks at a time: independent chains, few registers
-        split_row(x, y, next, seen);
+    constexpr int G = 2;           // column blocks at a time: independent chains, few registers
+    constexpr int P = RN / G * 6;  // MFMA pairs of a 16-k step
+    static_assert(RN % G == 0, "whole groups of column blocks");
+    bf8 b[G][3];
+    auto read_b = [&](int q, const unsigned char *bs) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j0 = 0; j0 < RN; j0 += G) {
-            bf8 b[G][3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q)
-#pragma unroll
-                for (int j = 0; j < G; ++j)
-                    b[j][q] = *reinterpret_cast<const bf8 *>(bs + (j0 + j) * 6144 + q * 1024 + lane * 16);
-#define MGC_MFMA(C, QA, QB)                          \
-    _Pragma("unroll") for (int j = 0; j < G; ++j)    \
-        C[j0 + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[QA], b[j][QB], C[j0 + j], 0, 0, 0);
-            MGC_MFMA(acc, 0, 0)
-            MGC_MFMA(cor, 2, 0)
-            MGC_MFMA(cor, 1, 0)
-            MGC_MFMA(cor, 1, 1)
-            MGC_MFMA(cor, 0, 1)
-            MGC_MFMA(cor, 0, 2)
-#undef MGC_MFMA
-        }
+        for (int j = 0; j < G; ++j) b[j][q] = *reinterpret_cast<const bf8 *>(bs + j * 6144 + q * 1024 + lane * 16);
     };
     // Stage kt: its copies and A loads have landed once at most the next stage's are outstanding
     // (R = 3), and every wave has read the slot that the new copies overwrite. Loads past the
     // end are masked, so the loop needs no tests.
+    //
+    // For a row-major A the order inside a stage is written out (sched_barrier): a group's B planes
+    // are read as the group before is done with its own, and the next step's A is split and the A
+    // of two stages on requested a quarter at a time between MFMA pairs. Left to the compiler, the
+    // split and the fragment waits stood in front of each step's MFMAs and the matrix cores were
+    // busy for 51% of the vocabulary projection (1024 x 768 x 50257 476 -> 448 us, BERT feed-forward
+    // b16 146 -> 139 us). The other forms need more address arithmetic between the loads, which
+    // the compiler places better (in this order: bottleneck b32 227 -> 236 us, 1003 x 515 x 1021 36 ->
+    // 43 us).
     int slot = 0;
-    bf8 a0[3], a1[3];
+    uint4_t a0[3], a1[3];
     auto stage = [&](f4 (&v)[4], f4 (&w)[4]) __attribute__((always_inline)) {
+        constexpr int QA[6] = {0, 2, 1, 1, 0, 0}, QB[6] = {0, 0, 0, 1, 1, 2};
         barrier_stage<(R - 2) * (DMA + 4)>();
-        copy_b(slot == 0 ? R - 1 : slot - 1);
         const unsigned char *const bs = smem + slot * SLOT;
-        step(a0, bs, v[2], v[3], a1);
-        load_a(v);
-        step(a1, bs + 3072, w[0], w[1], a0);
+        if constexpr (AMODE == AM_VEC) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) read_b(q, bs);
+            copy_b(slot == 0 ? R - 1 : slot - 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < 2 * P; ++t) {
+                const int s = t / P, q = t % P, i = t % 6, j0 = q / 6 * G;
+                const bf8 a = __builtin_bit_cast(bf8, s ? a1[QA[i]] : a0[QA[i]]);
+#pragma unroll
+                for (int j = 0; j < G; ++j) {
+                    floatx16 &c = i == 0 ? acc[j0 + j] : cor[j0 + j];
+                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[j][QB[i]], c, 0, 0, 0);
+                }
+                // planes 0, 1 and 2 of the next group after this group's last use of them
+                if ((i == 2 || i >= 4) && t + 6 - i < 2 * P) {
+                    const int n = t + 6 - i;
+                    read_b(i == 2 ? 0 : i - 3, bs + n / P * 3072 + n % P / 6 * G * 6144);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (q == (e * P + 2) / 4) {
+                        const f4 &x = s ? w[e >> 1] : v[2 + (e >> 1)];
+                        unsigned h, m, l;
+                        split3(x[2 * (e & 1)], x[2 * (e & 1) + 1], h, m, l);
+                        uint4_t(&next)[3] = s ? a0 : a1;
+                        next[0][e] = h;
+                        next[1][e] = m;
+                        next[2][e] = l;
+                        seen |= h;
+                    }
+                // v's first half was split in the stage before, its second half in this one's first step
+                if (t == P / 2) arow.load(p, ka, ka + 8 * lh, kend, v[0], v[1]);
+                if (t == P + P / 3) arow.load(p, ka, ka + 16 + 8 * lh, kend, v[2], v[3]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            copy_b(slot == 0 ? R - 1 : slot - 1);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                uint4_t(&a)[3] = s ? a1 : a0;
+                uint4_t(&next)[3] = s ? a0 : a1;
+                bf8 split[3];
+                split_row(s ? w[0] : v[2], s ? w[1] : v[3], split, seen);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) next[q] = __builtin_bit_cast(uint4_t, split[q]);
+#pragma unroll
+                for (int j0 = 0; j0 < RN; j0 += G) {
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) read_b(q, bs + s * 3072 + j0 * 6144);
+#pragma unroll
+                    for (int i = 0; i < 6; ++i)
+#pragma unroll
+                        for (int j = 0; j < G; ++j) {
+                            floatx16 &c = i == 0 ? acc[j0 + j] : cor[j0 + j];
+                            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8, a[QA[i]]), b[j][QB[i]], c, 0, 0, 0);
+                        }
+                }
+                if (s == 0) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) arow.load(p, ka, ka + 16 * h + 8 * lh, kend, v[2 * h], v[2 * h + 1]);
+                }
+            }
+        }
+        ka += BK;
         slot = slot == R - 1 ? 0 : slot + 1;
     };
 
@@ -380,7 +433,12 @@ __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
     copy_b(1);
     load_a(va[1]);
     asm volatile("" ::: "memory");
-    split_row(va[0][0], va[0][1], a0, seen);
+    {
+        bf8 first[3];
+        split_row(va[0][0], va[0][1], first, seen);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) a0[q] = __builtin_bit_cast(uint4_t, first[q]);
+    }
     for (int kt = nk >> 1; kt > 0; --kt) {
         stage(va[0], va[1]);
         stage(va[1], va[0]);
