@@ -3470,7 +3470,7 @@ static void gemm_launch(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const LnTai
         return;
     }
     if (split_fam) {
-        MGC_LAUNCH(x, pick_split(am_split, bm_s, bn_s), grid, dim3(bm_s == 32 ? 512 : 256), 0, p, static_cast<const unsigned char *>(planes),
+        MGC_LAUNCH(x, pick_split(am_split, bm_s, bn_s, p.kchunk), grid, dim3(bm_s == 32 ? 512 : 256), 0, p, static_cast<const unsigned char *>(planes),
                    plane_data_bytes(p.N, p.K), plane_kblocks(p.K));
     } else {
         MGC_LAUNCH(x, kern, grid, dim3(threads), 0, p);

@@ -14,8 +14,9 @@ enum { AM_LOOSE = 4, AM_TAP = 5 };
 constexpr bool is_conv(int am) { return am == AM_CONV_VEC || am == AM_TAP; }
 
 // The kernel for bm x bn tiles (128 x 128, 128 x 64, 32 x 64 or 32 x 32) of an A operand of form am
-// (AM_VEC, AM_CONV_VEC, AM_CAT, AM_LOOSE or AM_TAP).
-SplitKernel pick_split(int am, int bm, int bn);
+// (AM_VEC, AM_CONV_VEC, AM_CAT, AM_LOOSE or AM_TAP) and
+// kchunk k per workgroup.
+SplitKernel pick_split(int am, int bm, int bn, int kchunk);
 
 // Tile and K split of a GEMM on the bf16-split kernels; bm 0: the fp32 kernels are faster.
 struct SplitChoice {

@@ -260,7 +260,7 @@ __device__ __forceinline__ void fix_sums(const GemmDev &p, f4 &v, unsigned mark,
 //
 // A wave's 32 x 128 part has 2 x 64 accumulator registers, which two waves per SIMD (two
 // workgroups per CU) allow.
-template <int RN, int WAVES, int R, int AMODE>
+template <int RN, int WAVES, int R, int AMODE, bool ORDERED = false>
 __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
     gemm_split_kernel(const GemmDev p, const unsigned char *planes, long plane_bytes, int kblocks) {
     constexpr int BK = 32;
@@ -343,12 +343,12 @@ __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
     // (R = 3), and every wave has read the slot that the new copies overwrite. Loads past the
     // end are masked, so the loop needs no tests.
     //
-    // For a row-major A the order inside a stage is written out (sched_barrier): a group's B planes
-    // are read as the group before is done with its own, and the next step's A is split and the A
-    // of two stages on requested a quarter at a time between MFMA pairs. Left to the compiler, the
-    // split and the fragment waits stood in front of each step's MFMAs and the matrix cores were
+    // ORDERED (a row-major A): the order inside a stage is written out (sched_barrier). A group's B
+    // planes are read as the group before is done with its own, and the next step's A is split and
+    // the A of two stages on requested a quarter at a time between MFMA pairs. Left to the compiler,
+    // the split and the fragment waits stood in front of each step's MFMAs and the matrix cores were
     // busy for 51% of the vocabulary projection (1024 x 768 x 50257 476 -> 448 us, BERT feed-forward
-    // b16 146 -> 139 us). The other forms need more address arithmetic between the loads, which
+    // b16 146 -> 139 us). The other forms of A need more address arithmetic between the loads, which
     // the compiler places better (in this order: bottleneck b32 227 -> 236 us, 1003 x 515 x 1021 36 ->
     // 43 us).
     int slot = 0;
@@ -357,7 +357,7 @@ __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
         constexpr int QA[6] = {0, 2, 1, 1, 0, 0}, QB[6] = {0, 0, 0, 1, 1, 2};
         barrier_stage<(R - 2) * (DMA + 4)>();
         const unsigned char *const bs = smem + slot * SLOT;
-        if constexpr (AMODE == AM_VEC) {
+        if constexpr (ORDERED) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) read_b(q, bs);
             copy_b(slot == 0 ? R - 1 : slot - 1);
@@ -639,9 +639,12 @@ __global__ void __launch_bounds__(64 * WAVES)
     }
 }
 
+// The written-out order takes registers (164 instead of 128 at 64 columns, three waves a SIMD instead of
+// four), which short loops over many rows miss more than they gain: with K of 64 and 256 in this order
+// the bottleneck b32 takes 231 us instead of 228; K of 768 gains (the layers above).
 template <int RN>
-static SplitKernel pick(int am) {
-    return am == AM_VEC     ? &gemm_split_kernel<RN, 4, 3, AM_VEC>
+static SplitKernel pick(int am, int kchunk) {
+    return am == AM_VEC     ? (kchunk >= 512 ? &gemm_split_kernel<RN, 4, 3, AM_VEC, true> : &gemm_split_kernel<RN, 4, 3, AM_VEC>)
            : am == AM_CAT   ? &gemm_split_kernel<RN, 4, 3, AM_CAT>
            : am == AM_LOOSE ? &gemm_split_kernel<RN, 4, 3, AM_LOOSE>
            : am == AM_TAP   ? &gemm_split_kernel<RN, 4, 3, AM_TAP>
@@ -656,10 +659,10 @@ static SplitKernel pick_small(int am) {
                           : &gemm_split_small_kernel<RN, WAVES, AM_CONV_VEC>;
 }
 
-SplitKernel pick_split(int am, int bm, int bn) {
+SplitKernel pick_split(int am, int bm, int bn, int kchunk) {
     if (bm == 32 && am == AM_LOOSE) return &gemm_split_small_kernel<1, 8, AM_LOOSE>;  // bn 32 only: registers
     if (bm == 32) return bn == 64 ? pick_small<2, 8>(am) : pick_small<1, 8>(am);
-    return bn == 128 ? pick<4>(am) : pick<2>(am);
+    return bn == 128 ? pick<4>(am, kchunk) : pick<2>(am, kchunk);
 }
 
 }  // namespace mgc
