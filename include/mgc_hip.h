@@ -188,8 +188,9 @@ long mgc_hip_gemm_workspace(int M, int N, int K, int batch);
 /* GEMMs with a constant right-hand side on the bf16 matrix cores, in fp32 precision: B is laid
  * out once as three bf16 planes whose sums are its elements (24 bits), A is split the same way
  * when it is loaded, and six bf16 products accumulated in fp32 stand for each fp32 product.
- * Against 64 bits the result is no further off than mgc_hip_gemm's; infinities, NaN and
- * operands too small for the split are recomputed in fp32. No counterpart in the reference
+ * A product is within 2^-25 of its size, for operands of any size down to the smallest subnormal, and
+ * sums over many k are nearer 64 bits than mgc_hip_gemm's; sums that meet infinities or NaN, an operand
+ * of 2^112 or more, or that reach 2^96, are recomputed in fp32. No counterpart in the reference
  * (its mgc_gemm packs B for the CPU's caches, mgc_kernels.c:135-180).
  *
  *   mgc_hip_gemm_planes_bytes      bytes of the planes of a K x N right-hand side whose GEMMs over M

@@ -2834,8 +2834,7 @@ extern "C" long mgc_hip_gemm_planes_bytes(int M, int N, int K) {
     if (!split_choice(M, N, K, kAnyWorkspace, 0).bm && !split_choice(M, N, K, kAnyWorkspace, ln_split(M, N, K)).bm)
         return 0;
     const long bytes = plane_data_bytes(N, K);
-    // the planes, then a byte per column (whole blocks); buffer offsets end at 2 GiB
-    return bytes < 0x7fffffffL ? (bytes + plane_nblocks(N) * 32L + 255) / 256 * 256 : 0;
+    return bytes < 0x7fffffffL ? bytes : 0;  // buffer offsets end at 2 GiB
 }
 
 extern "C" long mgc_hip_gemm_planes_workspace(int M, int N, int K) {
@@ -2848,8 +2847,6 @@ extern "C" void mgc_hip_gemm_make_planes(mgc_hip_exec *x, const float *b, long l
     const int kb = plane_kblocks(K), nb = plane_nblocks(N);
     MGC_LAUNCH(x, split_planes_kernel, dim3(blocks_for((long)kb * nb * 64, 256, 16384)), dim3(256), 0, b, ldb, N, K, kb,
                nb, static_cast<uint4_t *>(planes));
-    MGC_LAUNCH(x, tiny_columns_kernel, dim3((unsigned)(nb * 32 / 4)), dim3(256), 0, b, ldb, N, K,
-               static_cast<unsigned char *>(planes) + plane_data_bytes(N, K), nb * 32);
 }
 
 extern "C" void mgc_hip_gemm_planes(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const void *planes) {

@@ -24,6 +24,5 @@ struct SplitChoice {
 };
 
 __global__ void split_planes_kernel(const float *b, long ldb, int N, int K, int kb, int nb, uint4_t *planes);
-__global__ void tiny_columns_kernel(const float *b, long ldb, int N, int K, unsigned char *flags, int nflags);
 
 }  // namespace mgc

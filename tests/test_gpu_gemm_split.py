@@ -223,6 +223,31 @@ def test_values_the_split_cannot_carry(runner, family):
     assert np.all(got[8][np.isfinite(b).all(1)] == 0.0)
 
 
+@pytest.mark.parametrize("family", FAMILIES)
+@pytest.mark.parametrize("k", [96, 99, 544])
+def test_small_numbers_beside_normal_ones(runner, family, k):
+    """Rows and columns that mix normal numbers with ones down to the smallest subnormal: where the other
+    operand is zero at the normal ones, the small ones are the whole sum, and it has fp32 precision.
+    The last term: up to eight waves' parts and their seven sums round to a subnormal's 2^-150 each (a
+    chain of fp32 products would at every k)."""
+    rng = np.random.default_rng(k)
+    m, n = 140, 72
+    a, b = rng.standard_normal((m, k)), rng.standard_normal((n, k))
+    half = rng.permutation(k) < k // 2
+    small = 2.0 ** rng.integers(-146, -104, (max(m, n), 1))  # one size to a row: nothing larger hides a loss
+    a[:70] = np.where(half, a[:70], a[:70] * small[:70])  # normal at `half`, small elsewhere
+    a[70:, half] = 0.0
+    b[:36, half] = 0.0
+    b[36:] = np.where(half, b[36:], b[36:] * small[36:n])
+    a, b = a.astype(np.float32), b.astype(np.float32)
+    assert np.any((a != 0) & (np.abs(a) < 2.0**-134)) and np.any((b != 0) & (np.abs(b) < 2.0**-134))
+    got = runner.gemm(family, a, b)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    want = a64 @ b64.T
+    assert np.all(np.abs(got - want) <= _bound(a64, b64, k) + 15 * 2.0**-150)
+    assert np.median(np.abs(want[:70, :36])) < 2.0**-100 and np.median(np.abs(want[70:, 36:])) < 2.0**-60
+
+
 def test_refusals(runner):
     """The families need planes and an A they can read; mgc_hip_gemm has none."""
     a, b = np.ones((128, 32), np.float32), np.ones((64, 32), np.float32)
