@@ -190,7 +190,7 @@ long mgc_hip_gemm_workspace(int M, int N, int K, int batch);
  * when it is loaded, and six bf16 products accumulated in fp32 stand for each fp32 product.
  * A product is within 2^-25 of its size, for operands of any size down to the smallest subnormal, and
  * sums over many k are nearer 64 bits than mgc_hip_gemm's; sums that meet infinities or NaN, an operand
- * of 2^112 or more, or that reach 2^96, are recomputed in fp32. No counterpart in the reference
+ * of 2^112 or more, or that reach 2^96, are recomputed in fp32 (32 rows of a tile at a time). No counterpart in the reference
  * (its mgc_gemm packs B for the CPU's caches, mgc_kernels.c:135-180).
  *
  *   mgc_hip_gemm_planes_bytes      bytes of the planes of a K x N right-hand side whose GEMMs over M

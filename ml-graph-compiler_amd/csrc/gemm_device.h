@@ -108,21 +108,16 @@ __device__ __forceinline__ f4 act4(f4 v, int act, float lo, float hi) {
 // pitch BN + 8 floats, leaves as 16-byte chunks with alpha, bias, residual and activation
 // applied, or raw into the split-K workspace. Each thread owns one fixed 16-byte column chunk
 // of the tile and the rows r0, r0 + RSTEP, ..., so the column bias is read once per thread.
-// Every one of the workgroup's THREADS threads calls it (no barrier inside). `fix` sees each chunk of raw sums with
-// its tile row and column before the epilogue (the bf16-split kernels replace sums there).
-struct NoFix {
-    __device__ __forceinline__ void operator()(f4 &, int, int, int) const {}
-};
-
-template <int BM, int BN, typename Fix = NoFix, int THREADS = 256>
+// Every one of the 256 threads calls it (no barrier inside).
+template <int BM, int BN>
 __device__ __forceinline__ void gemm_lds_to_global(const GemmDev &p, const float *Cs, int m0, int n0, int ks,
-                                                   long co, long ro, const Fix &fix = Fix()) {
+                                                   long co, long ro) {
     constexpr int LDC = BN + 8;
     const f4 zero4 = {0.f, 0.f, 0.f, 0.f};
     const int tid = threadIdx.x;
     constexpr int C4 = BN / 4;
-    static_assert(THREADS % C4 == 0, "column chunks must divide the workgroup");
-    constexpr int RSTEP = THREADS / C4;
+    static_assert(256 % C4 == 0, "column chunks must divide the workgroup");
+    constexpr int RSTEP = 256 / C4;
     constexpr int ITERS = BM / RSTEP;
     constexpr int G = ITERS < 4 ? ITERS : 4;
     // Scalars read once: keeps the compiler from copying the argument block to scratch.
@@ -174,7 +169,6 @@ __device__ __forceinline__ void gemm_lds_to_global(const GemmDev &p, const float
             const int row = m0 + rl;
             if (row >= M) break;
             f4 v = *reinterpret_cast<const f4 *>(&Cs[rl * LDC + cl]);
-            fix(v, rl, cl, ncol);
             float *dst = cbase + (long)row * ldc + col;
             if (!split_out) {
                 v = v * alpha + cbias;

@@ -13,6 +13,7 @@ arithmetic has them, rows or columns below 2^-95 keep fp32 precision.
 from __future__ import annotations
 
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -193,11 +194,12 @@ def test_concatenated_k(runner, family):
 
 
 @pytest.mark.parametrize("family", FAMILIES)
-def test_values_the_split_cannot_carry(runner, family):
+@pytest.mark.parametrize("k", [96, 99, 544, 1060])
+def test_values_the_split_cannot_carry(runner, family, k):
     """Infinities, NaN, overflow and the largest floats as fp32 has them; tiny rows and columns to
     fp32 precision; zeros exact; everything else in the same tiles untouched."""
     rng = np.random.default_rng(9)
-    m, n, k = 140, 72, 96
+    m, n = 140, 72
     a = rng.standard_normal((m, k)).astype(np.float32)
     b = rng.choice([0.5, -2.0, 1.0, 0.25, -1.5], (n, k)).astype(np.float32)  # exact in bf16: zero low parts
     a[3, 5] = np.inf
@@ -209,6 +211,7 @@ def test_values_the_split_cannot_carry(runner, family):
     a[9] *= np.float32(2.0**-120)
     a[130] *= np.float32(2.0**-100)
     b[11, 3] = np.inf
+    b[11, 10] = 0.5  # a[7, 10] times it is finite: an overflow and an infinity of other signs are NaN in one order only
     b[12] *= np.float32(2.0**-118)
     got = runner.gemm(family, a, b)
     with np.errstate(all="ignore"):
@@ -246,6 +249,33 @@ def test_small_numbers_beside_normal_ones(runner, family, k):
     want = a64 @ b64.T
     assert np.all(np.abs(got - want) <= _bound(a64, b64, k) + 15 * 2.0**-150)
     assert np.median(np.abs(want[:70, :36])) < 2.0**-100 and np.median(np.abs(want[70:, 36:])) < 2.0**-60
+
+
+def test_a_matrix_of_nan_costs_no_more_than_fp32_products(runner):
+    """Sums that are not finite are computed again, by the whole tile on the fp32 matrix cores: a product of
+    NaN alone takes a few times the finite one's time (six bf16 products cost 3/8 of the fp32 ones'), not
+    a serial loop's per element."""
+    m, n, k = 2048, 3072, 768
+    rng = np.random.default_rng(2)
+    b = rng.standard_normal((n, k)).astype(np.float32)
+    g = GemmArgs()
+    g.M, g.N, g.K, g.alpha = m, n, k, 1.0
+    g.a.rs, g.a.cs = k, 1
+    g.b.rs, g.b.cs = 1, k
+    g.b.p, planes = runner.planes(b)
+    g.c, g.ldc, g.kernel, g.split_k = runner.hip.empty(4 * m * n), n, FAMILIES["128x128"], 1
+    times = []
+    for a in (rng.standard_normal((m, k)).astype(np.float32), np.full((m, k), np.nan, np.float32)):
+        g.a.p = runner.hip.upload(a)
+        best = np.inf
+        for _ in range(5):
+            t = time.perf_counter()
+            assert runner.run(g, planes) == MGC_OK
+            best = min(best, time.perf_counter() - t)
+        times.append(best)
+    runner.hip.free()
+    print(f"2048 x 768 x 3072: finite {1e6 * times[0]:.0f} us, NaN {1e6 * times[1]:.0f} us", flush=True)
+    assert times[1] < 8 * times[0]
 
 
 def test_refusals(runner):
