@@ -2837,6 +2837,11 @@ extern "C" long mgc_hip_gemm_planes_bytes(int M, int N, int K) {
     return bytes < 0x7fffffffL ? bytes : 0;  // buffer offsets end at 2 GiB
 }
 
+extern "C" long mgc_hip_gemm_planes_wanted(int M, int N, int K, int layer_norm) {
+    if (M < 1 || N < 1 || K < 1 || !split_choice(M, N, K, kAnyWorkspace, layer_norm ? ln_split(M, N, K) : 0).bm) return 0;
+    return mgc_hip_gemm_planes_bytes(M, N, K);
+}
+
 extern "C" long mgc_hip_gemm_planes_workspace(int M, int N, int K) {
     if (!mgc_hip_gemm_planes_bytes(M, N, K)) return 0;
     const SplitChoice c = split_choice(M, N, K, kAnyWorkspace, 0);

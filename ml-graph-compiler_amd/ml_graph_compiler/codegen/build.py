@@ -114,6 +114,8 @@ def load_kernel_library() -> ctypes.CDLL:
         for fn in (lib.mgc_hip_gemm_planes_bytes, lib.mgc_hip_gemm_planes_workspace):
             fn.restype = ctypes.c_long
             fn.argtypes = [ctypes.c_int] * 3
+        lib.mgc_hip_gemm_planes_wanted.restype = ctypes.c_long
+        lib.mgc_hip_gemm_planes_wanted.argtypes = [ctypes.c_int] * 4
         lib.mgc_hip_last_error.restype = ctypes.c_char_p
         lib.mgc_hip_version.restype = ctypes.c_char_p
         lib.mgc_hip_device_count.restype = ctypes.c_int
@@ -129,10 +131,14 @@ def gemm_workspace_floats(m: int, n: int, k: int, batch: int) -> int:
     return max(int(lib.mgc_hip_gemm_workspace(m, n, k, batch)), planes)
 
 
-def gemm_planes_bytes(m: int, n: int, k: int) -> int:
+def gemm_planes_bytes(m: int, n: int, k: int, layer_norm: bool | None = None) -> int:
     """Device bytes of the bf16 planes of a constant k x n right-hand side whose GEMM over m rows the
-    kernel library runs on the bf16 matrix cores (0: it keeps the fp32 kernels)."""
-    return int(load_kernel_library().mgc_hip_gemm_planes_bytes(m, n, k))
+    kernel library runs on the bf16 matrix cores (0: it keeps the fp32 kernels): with a LayerNorm tail,
+    without, or (None) either way."""
+    lib = load_kernel_library()
+    if layer_norm is None:
+        return int(lib.mgc_hip_gemm_planes_bytes(m, n, k))
+    return int(lib.mgc_hip_gemm_planes_wanted(m, n, k, int(layer_norm)))
 
 
 def gemm_layer_norm_workspace_floats(m: int, n: int, k: int) -> int:

@@ -639,7 +639,7 @@ class HipEmitter:
         profile: bool = False,
         gemm_workspace: Callable[[int, int, int, int], int] | None = None,
         gemm_ln_workspace: Callable[[int, int, int], int] | None = None,
-        gemm_planes: Callable[[int, int, int], int] | None = None,
+        gemm_planes: Callable[[int, int, int, bool], int] | None = None,
     ) -> None:
         unsupported = sorted({n.op for n in graph.nodes} - self.SUPPORTED)
         if unsupported:
@@ -1413,7 +1413,8 @@ class HipEmitter:
                 parts.append(f"g.batch_dims[{d}] = {dim}; g.a_bs[{d}] = {abs_}L; g.b_bs[{d}] = {bbs}L; g.c_bs[{d}] = {cbs}L; g.r_bs[{d}] = {rbs}L;")
         parts.append(f"g.workspace = {workspace}; g.workspace_floats = {workspace_floats}L;")
         parts += extra
-        planes = self._planes_ptr(m, n, k, b) if not batch and depthwise is None and mbconv is None else None
+        planes = (self._planes_ptr(m, n, k, b, layer_norm is not None)
+                  if not batch and depthwise is None and mbconv is None else None)
         if layer_norm is not None:
             scale, lbias, eps, out = layer_norm
             if planes is not None:
@@ -1448,14 +1449,14 @@ class HipEmitter:
         self._packed_off[spec[0]] = off
         return spec
 
-    def _planes_ptr(self, m: int, n: int, k: int, b: list[str]) -> str | None:
+    def _planes_ptr(self, m: int, n: int, k: int, b: list[str], layer_norm: bool) -> str | None:
         """The planes of a packed constant right-hand side, laid out once at init from the weights
         blob, or None when the library keeps this GEMM on its fp32 kernels. GEMMs that share a
         matrix share its planes."""
         off = self._packed_off.get(b[0]) if len(b) == 1 else None
         if off is None or self._gemm_planes is None:
             return None
-        nbytes = int(self._gemm_planes(m, n, k))
+        nbytes = int(self._gemm_planes(m, n, k, layer_norm))
         if nbytes <= 0:
             return None
         at = self._planes.get((off, n, k))
@@ -2355,7 +2356,7 @@ def generate_hip(
     profile: bool = False,
     gemm_workspace: Callable[[int, int, int, int], int] | None = None,
     gemm_ln_workspace: Callable[[int, int, int], int] | None = None,
-    gemm_planes: Callable[[int, int, int], int] | None = None,
+    gemm_planes: Callable[[int, int, int, bool], int] | None = None,
 ) -> GeneratedModel:
     """Generate the host source and weights blob of a scheduled graph for the hip backend.
     ``gemm_workspace`` / ``gemm_ln_workspace`` ask the kernel library for split-K workspace

@@ -4,6 +4,8 @@ from __future__ import annotations
 
 import re
 
+import numpy as np
+
 from ml_graph_compiler import builders
 from ml_graph_compiler.codegen import build as native
 from ml_graph_compiler.codegen.hip import generate_hip
@@ -42,3 +44,18 @@ def test_small_gemms_keep_the_fp32_kernels():
     for m, n, k in ((1, 768, 768), (128, 768, 768), (32, 1000, 2048), (2048, 768, 32), (0, 1, 1)):
         assert native.gemm_planes_bytes(m, n, k) == 0
     assert native.gemm_planes_bytes(2048, 3072, 768) >= 3072 * 768 * 6
+
+
+def test_planes_only_for_the_call_that_reads_them():
+    """1024 x 768 x 768 reads planes with a LayerNorm tail (a K split of two) but not alone."""
+    def graph(norm):
+        b = builders.GraphBuilder("dense", 1)
+        x = b.op1("MatMul", [b.input("x", "float32", (1024, 768)), b.const(np.ones((768, 768), np.float32))])
+        if norm:
+            x = b.op1("LayerNormalization", [x, b.const(np.ones(768, np.float32)), b.const(np.zeros(768, np.float32))], axis=-1)
+        return b.finish([("out", x)])
+
+    assert native.gemm_planes_bytes(1024, 768, 768) > 0
+    plain, tail = _generate(graph(False)), _generate(graph(True))
+    assert "planes" not in plain.source and plain.arena_bytes == _generate(graph(False), planes=False).arena_bytes
+    assert "mgc_hip_gemm_planes_layer_norm" in tail.source
