@@ -197,7 +197,9 @@ long mgc_hip_gemm_workspace(int M, int N, int K, int batch);
  *                                  rows, alone or with a LayerNorm tail, the library would run this
  *                                  way; 0 when it would not
  *   mgc_hip_gemm_planes_wanted     the same for mgc_hip_gemm_planes (layer_norm 0) or
- *                                  mgc_hip_gemm_planes_layer_norm (1) only
+ *                                  mgc_hip_gemm_planes_layer_norm (1) only, in a model that reads
+ *                                  weight_bytes of GEMM weights a forward: planes are 6 bytes a
+ *                                  weight, and tiles of few rows pay for them only near the caches
  *   mgc_hip_gemm_planes_workspace  workspace floats mgc_hip_gemm_planes wants for its K split
  *   mgc_hip_gemm_make_planes       writes the planes (256-byte aligned device memory) of b, N rows of
  *                                  K floats with row stride ldb, on x's stream
@@ -206,7 +208,7 @@ long mgc_hip_gemm_workspace(int M, int N, int K, int batch);
  *                                  where the planes cannot be used (unaligned operands, batches)
  *   mgc_hip_gemm_planes_layer_norm the same for mgc_hip_gemm_layer_norm (planes may be NULL) */
 long mgc_hip_gemm_planes_bytes(int M, int N, int K);
-long mgc_hip_gemm_planes_wanted(int M, int N, int K, int layer_norm);
+long mgc_hip_gemm_planes_wanted(int M, int N, int K, int layer_norm, long weight_bytes);
 long mgc_hip_gemm_planes_workspace(int M, int N, int K);
 void mgc_hip_gemm_make_planes(mgc_hip_exec *x, const float *b, long ldb, int N, int K, void *planes);
 void mgc_hip_gemm_planes(mgc_hip_exec *x, const mgc_hip_gemm_args *g, const void *planes);

@@ -2837,9 +2837,30 @@ extern "C" long mgc_hip_gemm_planes_bytes(int M, int N, int K) {
     return bytes < 0x7fffffffL ? bytes : 0;  // buffer offsets end at 2 GiB
 }
 
-extern "C" long mgc_hip_gemm_planes_wanted(int M, int N, int K, int layer_norm) {
-    if (M < 1 || N < 1 || K < 1 || !split_choice(M, N, K, kAnyWorkspace, layer_norm ? ln_split(M, N, K) : 0).bm) return 0;
-    return mgc_hip_gemm_planes_bytes(M, N, K);
+// Whether a GEMM of a model that reads `weight_bytes` of GEMM weights a forward wants planes. 128-row tiles
+// use each of a weight's 6 plane bytes (4 in fp32) often enough to win wherever the weights come from.
+// 32-row tiles win alone, with the weights in the L2s, and lose where they are read once a forward from
+// the last-level cache or memory. us a layer in a chain of equal layers, fp32 kernel / these:
+//   1200 x 256 x 256  0.8 MB of weights in all 6.68 / 6.78, 3.9 MB 6.82 / 6.98, 32 MB 6.58 / 7.06
+//   784 x 448 x 448   0.8 MB 8.94 / 8.14, 3.2 MB 8.78 / 9.23, 15 MB 9.09 / 9.72, 99 MB 8.91 / 9.51
+//   392 x 768 x 768   2.4 MB 11.4 / 10.5, 7.1 MB 11.3 / 11.1, 14 MB 11.3 / 11.4, 99 MB 11.4 / 11.7, 198 MB 11.4 / 12.4
+// Up to 256 rows (the 128 x 2304 x 768 and 128 x 3072 x 768 layers of 128-token encoders of width 768; fp32
+// tiles of 32 x 32 run two rounds there) they win until the planes leave no room in the 256 MB last-level
+// cache: us a forward, 113 MB (4 layers) 246.2 / 244.2, 142 MB (5) 306.0 / 303.7, 170 MB (6) 364.7 / 366.8,
+// 198 MB (7) 424.6 / 435.6, BERT-base 763 / 781, GPT-2 846 / 863. Long K hides the loads (ResNet-50 b4's
+// 3136 x 128 x 1152 layers 696 / 683 us a forward); ResNet-50 b1, whose five shapes here have K of 128 to
+// 384, 378 / 387. The element-by-element fp32 kernel (K % 4) and a few rows over more columns than 16 x 16 tiles
+// take lose by far more (split_choice).
+static bool planes_pay(const SplitChoice &c, int M, int N, int K, long weight_bytes) {
+    if (c.bm != 32 || K % 4 != 0 || (M <= 32 && N > 8192)) return c.bm != 0;
+    const long mb = 1000000;
+    return weight_bytes <= (K < 512 ? 2 * mb : K < 1024 && M > 256 ? 8 * mb : 160 * mb);
+}
+
+extern "C" long mgc_hip_gemm_planes_wanted(int M, int N, int K, int layer_norm, long weight_bytes) {
+    if (M < 1 || N < 1 || K < 1) return 0;
+    const SplitChoice c = split_choice(M, N, K, kAnyWorkspace, layer_norm ? ln_split(M, N, K) : 0);
+    return planes_pay(c, M, N, K, weight_bytes) ? mgc_hip_gemm_planes_bytes(M, N, K) : 0;
 }
 
 extern "C" long mgc_hip_gemm_planes_workspace(int M, int N, int K) {

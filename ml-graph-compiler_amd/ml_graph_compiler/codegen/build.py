@@ -115,7 +115,7 @@ def load_kernel_library() -> ctypes.CDLL:
             fn.restype = ctypes.c_long
             fn.argtypes = [ctypes.c_int] * 3
         lib.mgc_hip_gemm_planes_wanted.restype = ctypes.c_long
-        lib.mgc_hip_gemm_planes_wanted.argtypes = [ctypes.c_int] * 4
+        lib.mgc_hip_gemm_planes_wanted.argtypes = [ctypes.c_int] * 4 + [ctypes.c_long]
         lib.mgc_hip_last_error.restype = ctypes.c_char_p
         lib.mgc_hip_version.restype = ctypes.c_char_p
         lib.mgc_hip_device_count.restype = ctypes.c_int
@@ -131,14 +131,14 @@ def gemm_workspace_floats(m: int, n: int, k: int, batch: int) -> int:
     return max(int(lib.mgc_hip_gemm_workspace(m, n, k, batch)), planes)
 
 
-def gemm_planes_bytes(m: int, n: int, k: int, layer_norm: bool | None = None) -> int:
+def gemm_planes_bytes(m: int, n: int, k: int, layer_norm: bool | None = None, weight_bytes: int = 0) -> int:
     """Device bytes of the bf16 planes of a constant k x n right-hand side whose GEMM over m rows the
     kernel library runs on the bf16 matrix cores (0: it keeps the fp32 kernels): with a LayerNorm tail,
-    without, or (None) either way."""
+    without, or (None) either way, in a model that reads ``weight_bytes`` of GEMM weights a forward."""
     lib = load_kernel_library()
     if layer_norm is None:
         return int(lib.mgc_hip_gemm_planes_bytes(m, n, k))
-    return int(lib.mgc_hip_gemm_planes_wanted(m, n, k, int(layer_norm)))
+    return int(lib.mgc_hip_gemm_planes_wanted(m, n, k, int(layer_norm), weight_bytes))
 
 
 def gemm_layer_norm_workspace_floats(m: int, n: int, k: int) -> int:

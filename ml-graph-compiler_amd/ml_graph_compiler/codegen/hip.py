@@ -639,7 +639,7 @@ class HipEmitter:
         profile: bool = False,
         gemm_workspace: Callable[[int, int, int, int], int] | None = None,
         gemm_ln_workspace: Callable[[int, int, int], int] | None = None,
-        gemm_planes: Callable[[int, int, int, bool], int] | None = None,
+        gemm_planes: Callable[[int, int, int, bool, int], int] | None = None,
     ) -> None:
         unsupported = sorted({n.op for n in graph.nodes} - self.SUPPORTED)
         if unsupported:
@@ -655,6 +655,10 @@ class HipEmitter:
         self._gemm_planes = gemm_planes
         self._planes: dict[tuple[int, int, int], int] = {}
         self._planes_bytes = 0
+        # what a forward reads of constant GEMM and convolution weights, each matrix once
+        rhs = {id(n.input(1)): n.input(1) for n in graph.nodes
+               if n.op in ("Conv", "FusedConv", "Gemm", "FusedGemm", "MatMul") and n.input(1).is_constant}
+        self._gemm_weight_bytes = sum(v.tensor_type.nbytes for v in rhs.values())
         # id(last 1 x 1 conv) -> its projection shortcut, and the shortcuts' ids. The shortcut's
         # input is then read at the last conv's step, which the plan must keep it alive for.
         self._shortcut: dict[int, Node] = find_projection_shortcuts(graph) if FUSE_PROJECTION_SHORTCUT else {}
@@ -1456,7 +1460,7 @@ class HipEmitter:
         off = self._packed_off.get(b[0]) if len(b) == 1 else None
         if off is None or self._gemm_planes is None:
             return None
-        nbytes = int(self._gemm_planes(m, n, k, layer_norm))
+        nbytes = int(self._gemm_planes(m, n, k, layer_norm, self._gemm_weight_bytes))
         if nbytes <= 0:
             return None
         at = self._planes.get((off, n, k))
@@ -2356,7 +2360,7 @@ def generate_hip(
     profile: bool = False,
     gemm_workspace: Callable[[int, int, int, int], int] | None = None,
     gemm_ln_workspace: Callable[[int, int, int], int] | None = None,
-    gemm_planes: Callable[[int, int, int, bool], int] | None = None,
+    gemm_planes: Callable[[int, int, int, bool, int], int] | None = None,
 ) -> GeneratedModel:
     """Generate the host source and weights blob of a scheduled graph for the hip backend.
     ``gemm_workspace`` / ``gemm_ln_workspace`` ask the kernel library for split-K workspace

@@ -59,3 +59,26 @@ def test_planes_only_for_the_call_that_reads_them():
     plain, tail = _generate(graph(False)), _generate(graph(True))
     assert "planes" not in plain.source and plain.arena_bytes == _generate(graph(False), planes=False).arena_bytes
     assert "mgc_hip_gemm_planes_layer_norm" in tail.source
+
+
+def test_tiles_of_few_rows_read_planes_where_weights_stay_cached():
+    """32-row tiles read planes in models whose weights stay near: alone (784 x 512 x 384), up to 8 MB
+    (392 x 768 x 768), in an encoder of 113 MB of weights (128 x 2304 x 768) but not in one of 198 MB.
+    128-row tiles and the forms that replace the element-by-element kernel read them in every model."""
+    mb = 1000000
+    wants = lambda m, n, k, w: native.gemm_planes_bytes(m, n, k, False, w) > 0  # noqa: E731
+    assert [wants(784, 512, 384, w * mb) for w in (1, 2, 3, 102)] == [True, True, False, False]
+    assert [wants(392, 768, 768, w * mb) for w in (2, 8, 9, 102)] == [True, True, False, False]
+    assert [wants(128, 2304, 768, w * mb) for w in (7, 113, 160, 170, 340)] == [True, True, True, False, False]
+    assert all(wants(m, n, k, 500 * mb) for m, n, k in ((2048, 3072, 768), (1, 50257, 768), (1003, 1021, 515), (7, 2999, 77)))
+    seen = set()
+
+    def record(m, n, k, layer_norm, weight_bytes):
+        seen.add(weight_bytes)
+        return 0
+
+    graph = builders.resnet50(1)
+    optimize(graph, "O3")
+    schedule(graph)
+    generate_hip(graph, gemm_workspace=native.gemm_workspace_floats, gemm_planes=record)
+    assert len(seen) == 1 and 100 * mb < seen.pop() < 103 * mb  # 25.5 million weights
