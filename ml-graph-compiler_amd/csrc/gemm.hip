@@ -2951,9 +2951,6 @@ extern "C" int mgc_hip_gemm_noalloc(void *stream, const mgc_hip_gemm_args *g) {
     a.workspace_floats = MGC_HIP_NOALLOC_SCRATCH_FLOATS;
     mgc_hip_exec x{};
     x.stream = static_cast<hipStream_t>(stream);
-    // an error the caller left pending on this thread is not this call's: the launch check
-    // after each kernel reads hipGetLastError()
-    (void)hipGetLastError();
     gemm_launch(&x, &a, nullptr);
     if (!x.launch_error) return MGC_OK;
     // gemm_launch reports operands outside a kernel's limits as hipErrorInvalidValue

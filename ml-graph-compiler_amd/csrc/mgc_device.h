@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <tuple>
+
 #include "mgc_hip.h"
 
 // One model's execution context (opaque to generated code).
@@ -20,8 +22,8 @@ struct mgc_hip_exec {
 
 namespace mgc {
 
-// Record the first launch error of a pass; the runtime reports it as MGC_ERR_HIP.
-void note_launch(mgc_hip_exec *x);
+// Count a launch and record the first launch error of a pass; the runtime reports it as MGC_ERR_HIP.
+void note_launch(mgc_hip_exec *x, hipError_t err);
 void set_error(const char *where, hipError_t err);
 
 inline unsigned blocks_for(long n, int threads, long cap = 1L << 20) {
@@ -196,8 +198,20 @@ __device__ __forceinline__ double wave_sum_d(double v) {
 
 }  // namespace mgc
 
-#define MGC_LAUNCH(x, kernel, grid, block, shmem, ...)                                         \
-    do {                                                                                       \
-        hipLaunchKernelGGL(kernel, grid, block, shmem, (x)->stream, __VA_ARGS__);              \
-        mgc::note_launch(x);                                                                   \
-    } while (0)
+// Launch a kernel on x's stream. The status is the launch's own: hipGetLastError would also give, and
+// clear, whatever error the calling thread has pending from its other work.
+namespace mgc {
+template <typename... P, typename... A>
+inline void launch(mgc_hip_exec *x, void (*kernel)(P...), dim3 grid, dim3 block, unsigned shmem, const A &...args) {
+    static_assert(sizeof...(P) == sizeof...(A), "one argument for each kernel parameter");
+    std::tuple<P...> values(static_cast<P>(args)...);
+    std::apply(
+        [&](P &...v) {
+            void *ptrs[] = {static_cast<void *>(&v)...};
+            note_launch(x, hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, ptrs, shmem, x->stream));
+        },
+        values);
+}
+}  // namespace mgc
+
+#define MGC_LAUNCH(x, kernel, grid, block, shmem, ...) mgc::launch(x, kernel, grid, block, shmem, __VA_ARGS__)

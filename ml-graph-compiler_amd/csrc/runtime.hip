@@ -133,10 +133,10 @@ void set_error(const char *where, hipError_t err) {
     g_last_error = std::string(where) + ": " + hipGetErrorString(err);
 }
 
-void note_launch(mgc_hip_exec *x) {
+void note_launch(mgc_hip_exec *x, hipError_t err) {
     ++x->launches;
-    hipError_t err = hipGetLastError();
     if (err != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not left for the caller's next check
         if (!x->launch_error) x->launch_error = (int)err;
         set_error("kernel launch", err);
     }

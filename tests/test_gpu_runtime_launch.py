@@ -55,3 +55,25 @@ def test_every_way_gives_the_same(layers, hip_cache):
     finally:
         model.release()
         hip.free()
+
+
+def test_an_error_pending_on_the_thread_is_the_callers(hip_cache):
+    """Launching kernel by kernel neither reports nor clears an error that the calling thread left from
+    its other work (a failed hipSetDevice)."""
+    graph = builders.mlp()
+    feeds = builders.random_feeds(graph, 3)
+    optimize(graph, "O3")
+    schedule(graph)
+    model = compile_graph(graph, cache_dir=hip_cache, name="pending")
+    hip = Hip()
+    try:
+        first = model.run(feeds)
+        for _ in range(3):
+            code = hip.lib.hipSetDevice(1 << 20)
+            assert code != 0 and hip.lib.hipPeekAtLastError() == code
+            again = model.run(feeds)
+            for name, value in first.items():
+                np.testing.assert_array_equal(again[name], value)
+            assert hip.lib.hipGetLastError() == code
+    finally:
+        model.release()
