@@ -113,6 +113,12 @@ int finish(ModelState *s) {
     return MGC_ERR_GATHER_INDEX;
 }
 
+// Status of a call on the caller's buffers: after an error too nothing of it is left in flight on them.
+int settled(ModelState *s, int rc) {
+    if (rc != MGC_OK && rc != MGC_ERR_GATHER_INDEX) (void)hipStreamSynchronize(s->stream);
+    return rc;
+}
+
 // One forward on the staging buffers.
 int staged_forward(mgc_hip_model *m, ModelState *s) {
     std::vector<const void *> in(s->in_stage.begin(), s->in_stage.end());
@@ -303,22 +309,24 @@ static int check_ptrs(mgc_hip_model *m, unsigned char *A, const unsigned char *W
     return MGC_OK;
 }
 
-int mgc_hip_model_run(mgc_hip_model *m, const void *const *inputs, void *const *outputs,
-                      unsigned char *A, const unsigned char *W) {
-    int rc = check_ptrs(m, A, W);
-    if (rc) return rc;
-    ModelState *s = state(m);
+static int run_staged(mgc_hip_model *m, ModelState *s, const void *const *inputs, void *const *outputs) {
     for (int i = 0; i < m->n_inputs; ++i)
         if (m->input_bytes[i])
             MGC_CHECK(hipMemcpyAsync(s->in_stage[i], inputs[i], m->input_bytes[i],
                                      hipMemcpyHostToDevice, s->stream));
-    rc = staged_forward(m, s);
+    const int rc = staged_forward(m, s);
     if (rc) return rc;
     for (int j = 0; j < m->n_outputs; ++j)
         if (m->output_bytes[j])
             MGC_CHECK(hipMemcpyAsync(outputs[j], s->out_stage[j], m->output_bytes[j],
                                      hipMemcpyDeviceToHost, s->stream));
     return finish(s);
+}
+
+int mgc_hip_model_run(mgc_hip_model *m, const void *const *inputs, void *const *outputs,
+                      unsigned char *A, const unsigned char *W) {
+    const int rc = check_ptrs(m, A, W);
+    return rc ? rc : settled(state(m), run_staged(m, state(m), inputs, outputs));
 }
 
 int mgc_hip_model_run_device(mgc_hip_model *m, const void *const *inputs, void *const *outputs,
@@ -336,8 +344,7 @@ int mgc_hip_model_run_device(mgc_hip_model *m, const void *const *inputs, void *
     }
     s->device_key = key;
     rc = forward(m, s, inputs, outputs, again, &s->device_graph);
-    if (rc) return rc;
-    return finish(s);
+    return settled(s, rc ? rc : finish(s));
 }
 
 int mgc_hip_model_upload(mgc_hip_model *m, const void *const *inputs) {
@@ -366,14 +373,17 @@ int mgc_hip_model_sync(mgc_hip_model *m) {
     return finish(state(m));
 }
 
-int mgc_hip_model_download(mgc_hip_model *m, void *const *outputs) {
-    if (!m || !m->state) return MGC_ERR_ARGS;
-    ModelState *s = state(m);
+static int download(mgc_hip_model *m, ModelState *s, void *const *outputs) {
     for (int j = 0; j < m->n_outputs; ++j)
         if (m->output_bytes[j])
             MGC_CHECK(hipMemcpyAsync(outputs[j], s->out_stage[j], m->output_bytes[j],
                                      hipMemcpyDeviceToHost, s->stream));
     return finish(s);
+}
+
+int mgc_hip_model_download(mgc_hip_model *m, void *const *outputs) {
+    if (!m || !m->state) return MGC_ERR_ARGS;
+    return settled(state(m), download(m, state(m), outputs));
 }
 
 double mgc_hip_model_time_graph(mgc_hip_model *m, int replays) {

@@ -9,8 +9,9 @@ import pytest
 
 from capi import Hip
 from ml_graph_compiler import builders
-from ml_graph_compiler.codegen import compile_graph
-from ml_graph_compiler.errors import GraphError
+from ml_graph_compiler.codegen import compile_graph, runtime_lib
+from ml_graph_compiler.codegen.hip import generate_hip
+from ml_graph_compiler.errors import CodegenError, GraphError
 from ml_graph_compiler.passes import optimize
 from ml_graph_compiler.schedule import schedule
 
@@ -77,3 +78,42 @@ def test_an_error_pending_on_the_thread_is_the_callers(hip_cache):
             assert hip.lib.hipGetLastError() == code
     finally:
         model.release()
+
+
+def test_nothing_is_in_flight_after_a_failed_forward(hip_cache, monkeypatch):
+    """A forward whose last launch is refused returns once the ones before it are done with the
+    caller's buffers."""
+    n = 4096
+    b = builders.GraphBuilder("half", 1)
+    x = b.input("x", "float32", (n, n))
+    y = b.op1("MatMul", [x, x])
+    graph = b.finish([("out", b.op1("MatMul", [y, x]))])
+    optimize(graph, "O3")
+    schedule(graph)
+
+    def refused(*args, **kwargs):  # the same forward, then a GEMM of an unknown kernel family
+        gen = generate_hip(*args, **kwargs)
+        end = gen.source.rindex("mgc_hip_gemm(x, &g);")
+        call = "mgc_hip_gemm(x, &g); g.kernel = 99; mgc_hip_gemm(x, &g);"
+        gen.source = gen.source[:end] + call + gen.source[end + len("mgc_hip_gemm(x, &g);"):]
+        return gen
+
+    model = compile_graph(graph, cache_dir=hip_cache, name="whole")
+    monkeypatch.setattr(runtime_lib, "generate_hip", refused)
+    failing = compile_graph(graph, cache_dir=hip_cache, name="half")
+    hip = Hip()
+    try:
+        pin = hip.upload(np.random.default_rng(1).standard_normal((n, n), dtype=np.float32))
+        want, out = hip.empty(4 * n * n), hip.empty(4 * n * n)
+        model.run_device([pin], [want])
+        for _ in range(3):
+            with pytest.raises(CodegenError):
+                failing.run_device([pin], [out])
+            got = np.empty((n,), np.float32)  # the last row, without waiting for other streams
+            hip.check(hip.lib.hipMemcpy(got.ctypes.data, out + 4 * n * (n - 1), got.nbytes, 2), "hipMemcpy D2H")
+            np.testing.assert_array_equal(got, hip.download(want, (n, n))[-1])
+            hip.put(out, np.full((n, n), np.nan, np.float32))
+    finally:
+        model.release()
+        failing.release()
+        hip.free()
