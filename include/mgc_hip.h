@@ -175,7 +175,8 @@ enum {
     /* mgc_hip_gemm_planes only: fp32 products on the bf16 matrix cores (gemm_split_kernel), by tile */
     MGC_GEMM_SPLIT_128X128 = 8,
     MGC_GEMM_SPLIT_128X64 = 9,
-    MGC_GEMM_SPLIT_32X64 = 10, /* K dealt to eight waves (gemm_split_small_kernel) */
+    MGC_GEMM_SPLIT_32X64 = 10, /* K dealt to eight waves (gemm_split_small_kernel); an A of rows that are only
+                                  4-byte aligned runs as 32X32 */
     MGC_GEMM_SPLIT_32X32 = 11
 };
 

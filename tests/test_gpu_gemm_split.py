@@ -107,8 +107,9 @@ def _check(got, a64, b64, bias=None, bias_mode=0, res=None, alpha=1.0, beta=1.0,
     assert np.all(np.abs(got - y) <= scale), float(np.max(np.abs(got - y) / scale))
 
 
-@pytest.mark.parametrize("family", FAMILIES)
-@pytest.mark.parametrize("k", [4, 16, 28, 32, 36, 64, 68, 100, 260, 1028, 5, 7, 30, 33, 65, 99, 259])
+# rows of K % 4 have no 32 x 64 form (32 x 32 tiles run instead)
+@pytest.mark.parametrize("family,k", [(f, k) for k in (4, 16, 28, 32, 36, 64, 68, 100, 260, 1028, 5, 7, 30, 33, 65, 99, 259)
+                                      for f in FAMILIES if f != "32x64" or k % 4 == 0])
 def test_shapes(runner, family, k):
     """Rows and columns at the tiles' edges, K at the stages', every epilogue and K splits."""
     rng = np.random.default_rng(k)
@@ -122,6 +123,60 @@ def test_shapes(runner, family, k):
         split = (1, 2, 3)[i % 3] if k >= 64 else 1
         got = runner.gemm(family, a, b, split=split, **ep)
         _check(got, a.astype(np.float64), b.astype(np.float64), **ep)
+
+
+def _split(x: np.ndarray) -> list[np.ndarray]:
+    """The three bf16 parts of floats, largest first, in float64."""
+    parts, rest = [], x.astype(np.float32)
+    for _ in range(3):
+        bits = rest.view(np.uint32)
+        part = ((bits + 0x7FFF + ((bits >> 16) & 1)) & np.uint32(0xFFFF0000)).view(np.float32)  # nearest, ties to even
+        parts.append(part.astype(np.float64))
+        rest = rest - part
+    assert not rest.any()
+    return parts
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+@pytest.mark.parametrize("k", [96, 99, 512, 540, 1056, 1060, 2076])
+def test_every_product_of_the_split(runner, family, k):
+    """Sums of four products in a long K, spread over the stages, their halves and a last partial stage: few
+    enough roundings to see any one of the six bf16 products missing anywhere. A leading sum and the
+    corrections round at most twice 2^-24 of the sum per product and once where they meet, and the
+    dropped products are 2^-25: 10 x 2^-24 S. K of 512 and more runs the main loop with the written-out order,
+    for the small tiles every wave's share of K."""
+    rng = np.random.default_rng(k)
+    m, n, t = 140, 136, 4
+    for sparse_a in (True, False):
+        shape, dense = ((m, k), (n, k)) if sparse_a else ((n, k), (m, k))
+        thin = np.zeros(shape, np.float32)
+        at = np.stack([rng.permutation(k)[:t] for _ in range(shape[0])])
+        at[: shape[0] // 2, 0] = k - 1 - np.arange(shape[0] // 2) % 36  # the last stage and the one before
+        np.put_along_axis(thin, at, rng.uniform(1.0, 2.0, at.shape).astype(np.float32), 1)
+        full = (rng.uniform(1.0, 2.0, dense) * rng.choice([-1.0, 1.0], dense)).astype(np.float32)
+        a, b = (thin, full) if sparse_a else (full, thin)
+        got = runner.gemm(family, a, b)
+        a64, b64 = a.astype(np.float64), b.astype(np.float64)
+        bound = 10 * 2.0**-24 * (np.abs(a64) @ np.abs(b64).T)
+        assert np.all(np.abs(got - a64 @ b64.T) <= bound)
+        pa, pb = _split(a), _split(b)
+        for i, j in ((0, 0), (0, 1), (1, 0), (0, 2), (1, 1), (2, 0)):  # what the bound sees
+            lost = np.abs(pa[i] @ pb[j].T)
+            assert np.mean(lost > 2 * bound) > 0.02, (i, j)
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+@pytest.mark.parametrize("k", [36, 516])
+def test_rows_of_four_byte_alignment(runner, family, k):
+    """K a multiple of four, A four bytes off the 16-byte alignment."""
+    rng = np.random.default_rng(k)
+    a = rng.standard_normal((130, k)).astype(np.float32)
+    b = (rng.standard_normal((70, k)) * 0.1).astype(np.float32)
+
+    def fill(g):
+        g.a.p = runner.hip.upload(np.concatenate([[np.float32(np.nan)], a.ravel()])) + 4
+
+    _check(runner.gemm(family, a, b, fill=fill), a.astype(np.float64), b.astype(np.float64))
 
 
 def _im2col(x: np.ndarray, kh: int, stride: int, pad: int) -> np.ndarray:
