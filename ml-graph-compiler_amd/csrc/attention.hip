@@ -685,8 +685,9 @@ extern "C" void mgc_hip_attention(mgc_hip_exec *x, const mgc_hip_attention_args 
     // Fewer (batch, head, 64-query) blocks than CUs and at least two key blocks: two groups of
     // four waves per workgroup take alternate key blocks and combine at the end (one workgroup
     // per CU then: the groups' tiles take 122 KB of LDS). With a causal mask up to two blocks a
-    // CU too where the sequences are long: all of them are resident at once, so the launch takes
-    // as long as the last query block, which meets every key block (us a layer, one group / two:
+    // CU too where the sequences are long: the second half of the query blocks, the short ones, start
+    // as the first end, and the launch takes about as long as the longest, which meets every key block
+    // and in two groups takes half the steps (us a layer, one group / two:
     // 384 blocks of 16 key blocks 190 / 162, 480 of 16 214 / 196, 384 of 8 165 / 158; 480 of 5 135 / 140,
     // 768 of 16 251 / 271).
     const int kblocks = (a->Skv + ATT_BK - 1) / ATT_BK;

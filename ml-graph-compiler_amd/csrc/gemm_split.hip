@@ -17,8 +17,8 @@
 // bit of every fp32 number, subnormals too, at 2^-133 or above (the MFMA keeps bf16 and fp32 subnormals),
 // and the sums are multiplied by 2^-32. That is one multiplication per element of A (marking rows and columns of
 // small numbers instead cost an instruction per two elements, and a small number beside normal ones
-// escaped it): ResNet-50 b32 2180 -> 2147 us, the vocabulary projection 444 -> 449, the 1003 x 515 x 1021
-// layer 36.0 -> 36.9.
+// escaped it): with the recomputation below, ResNet-50 b32 2212 -> 2169 us, the BERT feed-forward b16
+// 137.9 -> 135.9, the vocabulary projection, whose MFMAs wait for the split of A, 446 -> 451.
 //
 // Sums that are not finite (an infinite or NaN operand, operands of 2^112 or sums of 2^96 on, which the
 // scaled split overflows to infinities and NaN) are recomputed in fp32 from the operands: a wave that
@@ -345,9 +345,8 @@ __global__ void __launch_bounds__(64 * WAVES, RN >= 4 ? 2 : 3)
     // ORDERED (a row-major A): the order inside a stage is written out (sched_barrier). A group's B
     // planes are read as the group before is done with its own, and the next step's A is split and
     // the A of two stages on requested a quarter at a time between MFMA pairs. Left to the compiler,
-    // the split and the fragment waits stood in front of each step's MFMAs and the matrix cores were
-    // busy for 51% of the vocabulary projection (1024 x 768 x 50257 476 -> 448 us, BERT feed-forward
-    // b16 146 -> 139 us). The other forms of A need more address arithmetic between the loads, which
+    // the split and the fragment waits stood in front of each step's MFMAs (1024 x 768 x 50257 476 -> 448 us,
+    // BERT feed-forward b16 146 -> 139 us). The other forms of A need more address arithmetic between the loads, which
     // the compiler places better (in this order: bottleneck b32 227 -> 236 us, 1003 x 515 x 1021 36 ->
     // 43 us).
     int slot = 0;

@@ -2,11 +2,15 @@
 // captured into a hipGraph and replayed, a short one launched kernel by kernel, an error flag for
 // Gather in pinned host memory (zeroed at init, cleared again only after a check finds it set).
 //
-// Starting a graph costs the host 21 us however small it is, a launch 2.4 to 3 us (from the call to
-// the end of the wait, empty kernels: 1 kernel 32 us as a graph and 11 us launched, 4 kernels 33 and
-// 19 us, 20 kernels 47 and 83 us), so forwards of up to kEager launches take no graph. A longer one
-// is captured when it runs on the same buffers a second time: capturing costs more than it saves
-// on buffers that are used once. Kernels write the flag straight into host memory, so a call ends
+// Starting a graph costs the host 21 us however small it is, a launch 2.4 to 3 us, most of it while
+// earlier kernels run, so forwards of up to kEager launches take no graph. A call with n dependent
+// dense layers, us as a graph / launched: of 4 x 32 x 32, which the host's launches bound,
+//   n = 4 32.1 / 25.6, 6 34.6 / 32.8, 8 40.5 / 40.3-43.6, 10 46.4 / 47.5, 12 52.6 / 52.8-53.7, 16 64.1 / 66-68,
+//   20 78.4 / 80-82
+// and of 128 x 768 x 768 (6 us each), which hide them: n = 4 42.3 / 36.4, 8 68.2 / 60.6, 12 92.1 / 85.2,
+// 16 117.1 / 109.7, 24 166.0 / 158.8. kEager is where the smallest kernels break even, within 1 to 3 us from 8
+// launches on. A longer forward is captured when it runs on the same buffers a second time: capturing
+// costs more than it saves on buffers that are used once. Kernels write the flag straight into host memory, so a call ends
 // with the stream's synchronization; copying a device flag back took another 12 us. One call of a
 // four-kernel forward: 49 -> 25 us.
 //
