@@ -2,12 +2,13 @@
 """Benchmark of the hip backend: ResNet-50 fp32 img/s on one MI355X.
 
 A "step" is one forward pass of the compiled model over one batch of synthetic input (seeded
-N(0,1) images, He-normal weights, BatchNorm folded at -O3), replayed as the captured hipGraph
-with inputs already resident in HBM. The timed region is exactly ``--steps`` replays between two
-stream synchronizations (wall clock, cross-checked with hipEvents on the model stream).
+N(0,1) images, He-normal weights, BatchNorm folded at -O3) with inputs already resident in HBM: a
+long forward is a replayed hipGraph, one of a few kernels is launched kernel by kernel. The timed region
+is exactly ``--steps`` forwards between two stream synchronizations (wall clock, cross-checked with hipEvents on the model stream).
 
 Printed: ONE JSON line with the driver's fields plus
-* ``roofline``: the fp32 MFMA GEMM / implicit-GEMM convolution kernels (all conv and FC nodes):
+* ``roofline``: the fp32 GEMM / implicit-GEMM convolution kernels (all conv and FC nodes), on the fp32
+  MFMAs or as six bf16 products (``peak``: those kernels' own, time-weighted; ``of_fp32_mfma_peak``):
   algorithmic FLOPs per launch (ops.flops of the node, 2 per MAC) over the kernel's average
   duration in graph replays, measured in the run by a rocprofv3 --kernel-trace child over
   ``--trace-probe`` (``duration_source`` says so; ``event_avg_launch_us`` is the eager
@@ -36,6 +37,7 @@ sys.path[:0] = [str(ROOT), str(ROOT / "ml-graph-compiler_amd")]
 import numpy as np  # noqa: E402
 
 MFMA_FP32_PEAK_TFLOPS = 157.3
+MFMA_BF16_PEAK_TFLOPS = 2500.0
 HBM_PEAK_GBS = 8000.0
 
 
@@ -156,7 +158,7 @@ def feeds_for(graph, seed: int = 0):
 
 
 def time_replays(model, steps: int) -> tuple[float, float]:
-    """(wall seconds, event milliseconds) of ``steps`` graph replays on resident inputs."""
+    """(wall seconds, event milliseconds) of ``steps`` forwards on resident inputs."""
     model.sync()
     t0 = time.perf_counter()
     model.launch(steps)
@@ -186,14 +188,16 @@ def gemm_roofline(graph, model, replays: int) -> dict:
     return {
         "bound": "mfma",
         "kernel": ("the fp32 GEMM family: every GEMM / implicit-GEMM convolution kernel (gemm_split and "
-                   "gemm_split_small, whose fp32 products are six on the bf16 MFMAs: ceiling 416 TFLOP/s; "
+                   "gemm_split_small, whose fp32 products are six on the bf16 MFMAs: 2500 / 6 = 417 TFLOP/s; "
                    "gemm_dma, gemm_dma_tail, gemm_dma_wsplit, gemm_dma_wsplit16, gemm_stream, gemm_mfma, "
-                   "gemm_dw, gemm_expand_dw, mbconv on the fp32 MFMAs, whose peak is given), split-K "
-                   "reductions apart"),
+                   "gemm_dw, gemm_expand_dw, mbconv on the fp32 MFMAs: 157.3 TFLOP/s), split-K reductions "
+                   "apart; peak is those kernels' own, weighted by the time each took in the kernel trace "
+                   "(the fp32 MFMAs' without a trace)"),
         "achieved": round(achieved, 2),
         "peak": MFMA_FP32_PEAK_TFLOPS,
         "unit": "TFLOP/s",
         "frac": round(achieved / MFMA_FP32_PEAK_TFLOPS, 4),
+        "of_fp32_mfma_peak": round(achieved / MFMA_FP32_PEAK_TFLOPS, 4),
         "traffic": None,
         "flops_per_launch": int(flops / max(launches, 1)),
         "avg_launch_us": round(1e6 * secs / max(launches, 1), 2),
@@ -367,6 +371,18 @@ def trace_probe(workload: str, batch: int, cache: Path) -> None:
     log(f"trace probe done: {TRACE_REPLAYS} graph replays")
 
 
+def _of_forward(name: str) -> bool:
+    """Whether a traced kernel belongs to a forward: not the runtime's own blit kernels (uploads), nor
+    the layout of the weights' bf16 planes, which runs once when a model is loaded."""
+    return not name.startswith("__amd_rocclr") and "split_planes_kernel" not in name
+
+
+def _mfma_peak(name: str) -> float:
+    """TFLOP/s of fp32 products that a GEMM kernel's matrix instructions allow: the bf16-split kernels
+    spend six bf16 products on each."""
+    return MFMA_BF16_PEAK_TFLOPS / 6 if "gemm_split_" in name else MFMA_FP32_PEAK_TFLOPS
+
+
 def _is_gemm_kernel(name: str) -> bool:
     """The GEMM family: every GEMM / implicit-GEMM kernel (the whole-block mbconv kernel is the
     projection GEMM with its producers fused), not the split-K reductions."""
@@ -399,10 +415,11 @@ def traced_gemm_launch(workload: str, batch: int, cache: Path) -> dict | None:
             for r in csv.DictReader(open(f)):
                 rows.append((r["Kernel_Name"], (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) * 1e-3))
         gemm = [us for name, us in rows if _is_gemm_kernel(name)]
+        peak = sum(us * _mfma_peak(name) for name, us in rows if _is_gemm_kernel(name)) / max(sum(gemm), 1e-9)
         red = [us for name, us in rows if "splitk" in name]
         if not gemm:
             raise RuntimeError(f"no GEMM dispatches traced (rc {proc.returncode}): {proc.stderr[-300:]}")
-        return {"launches": len(gemm), "avg_us": sum(gemm) / len(gemm),
+        return {"launches": len(gemm), "peak": peak, "avg_us": sum(gemm) / len(gemm),
                 "avg_us_with_reductions": (sum(gemm) + sum(red)) / len(gemm), "reductions": len(red)}
     except Exception as exc:
         log(f"kernel trace failed: {exc}")
@@ -526,8 +543,8 @@ def hbm_summary(fetch_dir: Path, write_dir: Path, trace_dir: Path, workload: str
         i = next(k for k, r in enumerate(rows) if "copy_kernel" in r[1 if len(r) == 3 else 0])
         return rows[i + 1:]
 
-    def kernels_only(rows):  # the runtime's own blit kernels (uploads) are not the model's
-        return [r for r in rows if not r[1 if len(r) == 3 else 0].startswith("__amd_rocclr")]
+    def kernels_only(rows):
+        return [r for r in rows if _of_forward(r[1 if len(r) == 3 else 0])]
 
     fetch, write = kernels_only(from_calibration(fetch)), kernels_only(from_calibration(write))
     trace = kernels_only(from_calibration(trace))
@@ -603,13 +620,13 @@ def hbm_summary(fetch_dir: Path, write_dir: Path, trace_dir: Path, workload: str
 
 MI355X_CLOCK_HZ = 2.4e9
 MI355X_SIMDS = 256 * 4
-MFMA_COUNTERS = "SQ_INSTS_VALU_MFMA_MOPS_F32 SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CU_CYCLES GRBM_GUI_ACTIVE"
+MFMA_COUNTERS = "SQ_INSTS_VALU_MFMA_MOPS_F32 SQ_INSTS_VALU_MFMA_MOPS_BF16 SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CU_CYCLES GRBM_GUI_ACTIVE"
 
 
 def kernel_summary(trace_dir: Path, workload: str, batch: int) -> str:
     """Per-kernel durations of graph replays: a rocprofv3 --kernel-trace run of --trace-probe
-    (3 warmup + TRACE_REPLAYS replays, nothing else on the GPU apart from the upload copies),
-    averaged per forward, with the GEMM family's algorithmic TFLOP/s (node FLOPs from the
+    (3 warmup + TRACE_REPLAYS replays; the upload copies and the planes' layout at load are left
+    out), averaged per forward, with the GEMM family's algorithmic TFLOP/s (node FLOPs from the
     compiled graph, a fused projection shortcut or depthwise convolution counted at the launch
     that computes it)."""
     import csv
@@ -620,7 +637,7 @@ def kernel_summary(trace_dir: Path, workload: str, batch: int) -> str:
     rows = []
     for f in sorted(trace_dir.rglob("*kernel_trace.csv")):
         for r in csv.DictReader(open(f)):
-            if r["Kernel_Name"].startswith("__amd_rocclr"):
+            if not _of_forward(r["Kernel_Name"]):
                 continue
             rows.append((int(r["Dispatch_Id"]), _short_kernel(r["Kernel_Name"]),
                          (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) * 1e-9))
@@ -656,7 +673,7 @@ def kernel_summary(trace_dir: Path, workload: str, batch: int) -> str:
         f"python3 bench.py --kernel-summary gpurun_out/kt_{workload}_b{batch} --workload {workload} --batch {batch}",
         "```",
         "",
-        f"The probe replays the captured forward {forwards} times (3 warmup + {TRACE_REPLAYS}) on resident inputs; "
+        f"The probe runs the forward {forwards} times (3 warmup + {TRACE_REPLAYS}; a long one as a replayed graph) on resident inputs; "
         f"durations are the kernel trace's end - start of each dispatch, averaged per forward. Kernel time per "
         f"forward: {total * 1e6:.1f} us in {len(rows) / forwards:.0f} launches.",
         "",
@@ -668,10 +685,14 @@ def kernel_summary(trace_dir: Path, workload: str, batch: int) -> str:
                    f"{100 * sec / forwards / total:.1f} |")
     if gemm_n:
         tf = gemm_flops / gemm_sec / 1e12
+        peak = sum(sec * _mfma_peak(name) for _, name, sec in rows if _is_gemm_kernel(name)) / forwards / gemm_sec
         out += ["", f"GEMM family (every GEMM / implicit-GEMM kernel, split-K reductions apart): {gemm_n:g} launches "
                     f"per forward, {gemm_sec / gemm_n * 1e6:.2f} us average, {gemm_flops / 1e9:.2f} GFLOP algorithmic "
                     f"per forward -> {tf:.1f} TFLOP/s = {100 * tf / MFMA_FP32_PEAK_TFLOPS:.1f}% of the "
-                    f"{MFMA_FP32_PEAK_TFLOPS} TFLOP/s fp32 MFMA peak."]
+                    f"{MFMA_FP32_PEAK_TFLOPS} TFLOP/s fp32 MFMA peak"
+                    + (f", {100 * tf / peak:.1f}% of the {peak:.0f} TFLOP/s that its kernels' own matrix "
+                       f"instructions allow (time-weighted; {MFMA_BF16_PEAK_TFLOPS / 6:.0f} for the bf16-split "
+                       f"kernels)." if peak > 1.001 * MFMA_FP32_PEAK_TFLOPS else ".")]
         stats = []
         for f in sorted(trace_dir.rglob("*kernel_stats.csv")):
             stats += [(r["Name"], int(r["Calls"]), float(r["TotalDurationNs"])) for r in csv.DictReader(open(f))]
@@ -687,9 +708,9 @@ def kernel_summary(trace_dir: Path, workload: str, batch: int) -> str:
 def mfma_summary(pmc_dir: Path, trace_dir: Path, workload: str, batch: int) -> str:
     """MFMA work and utilisation of every matrix-core dispatch of one eager forward: one counter
     run over --pmc-probe (MFMA_COUNTERS) and the kernel-trace run of the same program for
-    durations, matched by position and checked by name. SQ_INSTS_VALU_MFMA_MOPS_F32 counts fp32
-    MFMA work in units of 512 FLOP; SQ_VALU_MFMA_BUSY_CYCLES counts matrix-core busy cycles,
-    reported here per CU per GPU-active cycle (GRBM_GUI_ACTIVE)."""
+    durations, matched by position and checked by name. SQ_INSTS_VALU_MFMA_MOPS_F32 and _BF16 count
+    MFMA work in units of 512 FLOP, six bf16 ones to an fp32 one in the bf16-split kernels;
+    SQ_VALU_MFMA_BUSY_CYCLES counts matrix-core busy cycles."""
     import csv
 
     counters: dict[int, dict] = {}
@@ -707,7 +728,7 @@ def mfma_summary(pmc_dir: Path, trace_dir: Path, workload: str, batch: int) -> s
 
     def model_only(seq, name_of):
         i = next(k for k, r in enumerate(seq) if "copy_kernel" in name_of(r))
-        return [r for r in seq[i + 1:] if not name_of(r).startswith("__amd_rocclr")]
+        return [r for r in seq[i + 1:] if _of_forward(name_of(r))]
 
     rows = model_only(rows, lambda r: r["name"])
     trace = model_only(trace, lambda r: r[1])
@@ -716,7 +737,7 @@ def mfma_summary(pmc_dir: Path, trace_dir: Path, workload: str, batch: int) -> s
     fam: dict[str, list] = {}
     tot_flop = tot_sec = 0.0
     for r, (_, name, sec) in zip(rows, trace):
-        flop = 512.0 * r.get("SQ_INSTS_VALU_MFMA_MOPS_F32", 0.0)
+        flop = 512.0 * (r.get("SQ_INSTS_VALU_MFMA_MOPS_F32", 0.0) + r.get("SQ_INSTS_VALU_MFMA_MOPS_BF16", 0.0) / 6)
         if flop <= 0:
             continue
         busy = r.get("SQ_VALU_MFMA_BUSY_CYCLES", 0.0) / (sec * MI355X_CLOCK_HZ * MI355X_SIMDS)
@@ -740,9 +761,10 @@ def mfma_summary(pmc_dir: Path, trace_dir: Path, workload: str, batch: int) -> s
         f"python3 bench.py --mfma-summary gpurun_out/mfma_pmc gpurun_out/hbm_trace --workload {workload} --batch {batch}",
         "```",
         "",
-        "FLOP = 512 x SQ_INSTS_VALU_MFMA_MOPS_F32 (the fp32 MFMA work the matrix cores executed, "
-        "padding of partial tiles included); TFLOP/s = that over the traced duration; % of peak "
-        f"against {MFMA_FP32_PEAK_TFLOPS} TFLOP/s. MFMA busy = SQ_VALU_MFMA_BUSY_CYCLES over the "
+        "FLOP = 512 x (SQ_INSTS_VALU_MFMA_MOPS_F32 + SQ_INSTS_VALU_MFMA_MOPS_BF16 / 6) (the fp32 products the "
+        "matrix cores executed, six bf16 ones each in the gemm_split kernels, padding of partial tiles "
+        "included); TFLOP/s = that over the traced duration; % of peak against "
+        f"{MFMA_FP32_PEAK_TFLOPS} TFLOP/s, and {MFMA_BF16_PEAK_TFLOPS / 6:.0f} for the gemm_split kernels. MFMA busy = SQ_VALU_MFMA_BUSY_CYCLES over the "
         "traced duration x 2.4 GHz x 1024 SIMDs (256 CUs x 4), time-weighted: the fraction of "
         "matrix-core cycles in use. (GRBM_GUI_ACTIVE, summed over the 8 XCDs and stretched by the "
         "counter collection, is not used as the time base.)",
@@ -753,11 +775,11 @@ def mfma_summary(pmc_dir: Path, trace_dir: Path, workload: str, batch: int) -> s
     for name, (cnt, flop, sec, busy_sec) in sorted(fam.items(), key=lambda kv: -kv[1][2]):
         tf = flop / sec / 1e12
         out.append(f"| `{name}` | {cnt} | {flop / cnt / 1e9:.3f} | {sec / cnt * 1e6:.2f} | {tf:.1f} | "
-                   f"{100 * tf / MFMA_FP32_PEAK_TFLOPS:.1f} | {busy_sec / sec:.3f} |")
+                   f"{100 * tf / _mfma_peak(name):.1f} | {busy_sec / sec:.3f} |")
     if tot_sec > 0:
         tf = tot_flop / tot_sec / 1e12
         out += ["", f"All MFMA dispatches: {tot_flop / 1e9:.1f} GFLOP in {tot_sec * 1e6:.1f} us = {tf:.1f} TFLOP/s "
-                    f"({100 * tf / MFMA_FP32_PEAK_TFLOPS:.1f}% of peak)."]
+                    f"({100 * tf / MFMA_FP32_PEAK_TFLOPS:.1f}% of the fp32 MFMA peak)."]
         from ml_graph_compiler import ops
         from ml_graph_compiler.passes import optimize
 
@@ -866,7 +888,9 @@ def main() -> int:
         roof["event_avg_launch_us"] = roof["avg_launch_us"]
         roof["avg_launch_us"] = round(traced["avg_us"], 2)
         roof["achieved"] = round(flops / traced["avg_us"] / 1e6, 2)
-        roof["frac"] = round(roof["achieved"] / MFMA_FP32_PEAK_TFLOPS, 4)
+        roof["peak"] = round(traced["peak"], 1)
+        roof["frac"] = round(roof["achieved"] / traced["peak"], 4)
+        roof["of_fp32_mfma_peak"] = round(roof["achieved"] / MFMA_FP32_PEAK_TFLOPS, 4)
         roof["achieved_with_reductions"] = round(flops / traced["avg_us_with_reductions"] / 1e6, 2)
         roof["duration_source"] = (f"rocprofv3 --kernel-trace over {TRACE_REPLAYS} graph replays "
                                    f"({traced['launches']} GEMM dispatches, {traced['reductions']} split-K reductions)")
